@@ -122,7 +122,9 @@ hipError_t launch_attention_fwd(const mc_attn_desc& d, const void* q, const void
 // Delta per 64-query block (f32 [B, H, Sp/64, 2, 64], Sp = S rounded up to
 // 64) and, when the dK/dV kernel splits a K/V head's query heads into more
 // than one group (attn_dkdv_groups), the per-group dK / dV partials (f32
-// [B, Hkv, groups, S, D]). Generic path: Delta (f32 [B, H, S]) at lsd.
+// [B, Hkv, groups, S, D]). fp32 MFMA path: Delta (f32 [B, H, S]) at lsd and,
+// with more than one group (attention_f32_groups), the partials in the same
+// layout. Generic path: Delta at lsd.
 struct AttnBwdWs {
     size_t lsd, dk_part, dv_part;
     size_t dst;  // bf16 dS^T [B, H, S, ldst] for the dQ pass (attention_dq_from_ds), else unused
@@ -133,6 +135,21 @@ int attn_dkdv_groups(const mc_attn_desc& d);
 hipError_t launch_attention_bwd(const mc_attn_desc& d, const void* q, const void* k, const void* v,
                                 const float* mask, const void* o, const float* lse, const void* dout, void* dq,
                                 void* dk, void* dv, void* ws, hipStream_t stream);
+
+// fp32 on the matrix cores (attention_f32.hip): head dims that are a multiple
+// of 4 (rows of whole 16-byte vectors), at most 128.
+bool attention_f32_mfma(const mc_attn_desc& d);
+// Groups that a K/V head's query heads are split into for dK/dV: the smallest
+// divisor of H / Hkv that gives 1024 workgroups (four per CU), at most one
+// head per group. A function of the shape only, as the order of the sums is.
+int attention_f32_groups(const mc_attn_desc& d);
+hipError_t launch_attention_f32_fwd(const mc_attn_desc& d, const void* q, const void* k, const void* v,
+                                    const float* mask, void* o, float* lse, hipStream_t stream);
+// delta: [B, H, S]; dk_part, dv_part: [B, Hkv, groups, S, D], used when groups > 1.
+hipError_t launch_attention_f32_bwd(const mc_attn_desc& d, const void* q, const void* k, const void* v,
+                                    const float* mask, const void* o, const float* lse, const void* dout, void* dq,
+                                    void* dk, void* dv, float* delta, float* dk_part, float* dv_part,
+                                    hipStream_t stream);
 
 // --------------------------------------------------------------- AdamW
 // One launch of the AdamW kernel updates up to kAdamWSlots tensors; the
