@@ -689,6 +689,215 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma(int64_t M, int64_t N, F32Se
     }
 }
 
+// fp32 products of many tiles: a workgroup owns a 64 x 64 tile of C, its 4
+// waves a 32 x 32 MFMA tile each, and walks the first segment in steps of 32 k
+// through a ring of four 16 KB LDS stages filled by LDS-DMA. Step kt starts
+// with a wait for step kt + 1's loads and a barrier, requests step kt + 3 into
+// the stage of step kt - 1 and multiplies stage kt % 4; its last operand reads
+// already come from the next stage, so no MFMA waits for a barrier and an LDS
+// read in turn. A step's MFMAs take 0.43 us and a load from HBM about 1 us:
+// with one step in flight per workgroup the same tile ran at half the rate.
+// Row-major operands are staged as rows of 128 bytes with the chunk swizzle of
+// the bf16 GEMM; with NN the segment's B, stored [k][N], as k rows of 256
+// bytes, chunk c of row k in slot c ^ 8 ((k / 4) % 2), so that the two k rows
+// of an operand read fall on different banks.
+//
+// The rank-r columns (second segment, any alignment, the other B layout) are
+// requested into registers before the loop, 64 ranks at a time, and go through
+// the free stages after it.
+//
+// v_mfma_f32_32x32x2_f32 takes 64 cycles for 2 floats per lane and operand, so
+// what bounds the kernel is MFMA issue. Vector arithmetic does not overlap with
+// it, unlike with the bf16 MFMAs: 16 additions per step cost 0.05 us of the
+// step's 0.43, so the loop holds none but the partial sums below.
+//
+// Rounding: every sum_steps steps (about a twelfth of the reduction) are summed
+// on their own and added to the total, so the error stays below that of
+// gemm_f32_mfma's four chains over the whole reduction.
+template <bool NN>
+__global__ __launch_bounds__(256, 2) void gemm_f32_tiled(int64_t M, int64_t N, F32Seg s0, F32Seg s1,
+                                                         const float* __restrict__ bias, float* __restrict__ C,
+                                                         int64_t ldc, int tiles_m, int tiles_n) {
+    constexpr int BT = 64, BK = 32, STAGES = 4, LOADS = 4;
+    constexpr int TILE = BT * BK, STAGE = 2 * TILE;  // floats
+    __shared__ __attribute__((aligned(1024))) float sm[STAGES * STAGE];
+    const uint32_t sm_byte = (uint32_t)reinterpret_cast<uintptr_t>(sm);
+    const int lane = lane_id(), wave = wave_id(), tid = (int)threadIdx.x;
+    const int rc = lane & 31, h = lane >> 5, wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    int tm, tn;
+    tile_of((int)blockIdx.x, tiles_m, tiles_n, 4, tm, tn);
+    const int64_t m0 = (int64_t)__builtin_amdgcn_readfirstlane(tm) * BT;
+    const int64_t n0 = (int64_t)__builtin_amdgcn_readfirstlane(tn) * BT;
+    const int64_t mrows = M - m0 < BT ? M - m0 : BT, nrows = N - n0 < BT ? N - n0 : BT;
+    const int nk = (int)((s0.k + BK - 1) / BK), nfull = (int)(s0.k / BK);
+    const int sum_steps = nk < 24 ? 1 : nk < 96 ? nk / 12 : 8;
+    int next_sum = sum_steps - 1;
+
+    // the rank-r columns' first 64, in registers until the loop is done
+    const uint32_t lr = (uint32_t)tid >> 2, lk = 16u * ((uint32_t)tid & 3u);  // row-major: row, 16 k
+    const uint32_t kr = (uint32_t)tid >> 2, nc = 16u * ((uint32_t)tid & 3u);  // [k][N]: k row, 16 columns
+    const __amdgpu_buffer_rsrc_t ra1 = make_rsrc(s1.a + m0 * s1.lda, s1.k > 0 ? ((mrows - 1) * s1.lda + s1.k) * 4 : 0);
+    const __amdgpu_buffer_rsrc_t rb1 =
+        NN ? make_rsrc(s1.b + n0 * s1.ldb, s1.k > 0 ? ((nrows - 1) * s1.ldb + s1.k) * 4 : 0)
+           : make_rsrc(s1.b + n0, s1.k > 0 ? ((s1.k - 1) * s1.ldb + (N - n0)) * 4 : 0);
+    f32x4 ea[4], eb[4];
+    auto load_ext = [&](int64_t k0) {
+        const uint32_t oa = (lr * (uint32_t)s1.lda + (uint32_t)k0 + lk) * 4u;
+        const uint32_t ob = NN ? (lr * (uint32_t)s1.ldb + (uint32_t)k0 + lk) * 4u
+                               : (((uint32_t)k0 + kr) * (uint32_t)s1.ldb + nc) * 4u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            ea[i] = __builtin_bit_cast(f32x4, buf_load16(ra1, oa + 16u * i));
+            eb[i] = __builtin_bit_cast(f32x4, buf_load16(rb1, ob + 16u * i));
+        }
+    };
+    load_ext(0);
+
+    const i32x4 ra = rsrc_words(s0.a + m0 * s0.lda, ((mrows - 1) * s0.lda + s0.k) * 4);
+    const i32x4 rb = NN ? rsrc_words(s0.b + n0, ((s0.k - 1) * s0.ldb + (N - n0)) * 4)
+                        : rsrc_words(s0.b + n0 * s0.ldb, ((nrows - 1) * s0.ldb + s0.k) * 4);
+    // rows of 32 floats are rows of 64 bf16 to the DMA helpers
+    const uint32_t lda2 = 2u * (uint32_t)s0.lda, ldb2 = 2u * (uint32_t)s0.ldb;
+    TileOffsets<BT, 256, 64> offa, offb;
+    offa.init(lda2, tid);
+    uint32_t offk[2];  // NN: k rows 8 wave + 4 j + lane / 16
+    if constexpr (NN) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const uint32_t row = (uint32_t)(8 * wave + 4 * j + (lane >> 4));
+            offk[j] = (row * (uint32_t)s0.ldb + 4u * (uint32_t)((lane & 15) ^ (8 * j))) * 4u;
+        }
+    } else {
+        offb.init(ldb2, tid);
+    }
+    const uint32_t lds_wave = sm_byte + (uint32_t)wave * 2048u;
+    // Load i of the wave's four of step kt: two of A, two of B.
+    auto issue = [&](int kt, int stage, int i) {
+        const uint32_t base = lds_wave + (uint32_t)stage * (STAGE * 4);
+        const bool full = kt < nfull;
+        if (i < 2) {
+            if (full) dma_tile_full<BT, 256, 64, 2>(ra, base, offa, (uint32_t)kt * 64u, i);
+            else dma_tile<BT, 256, 64, 2>(ra, base - (uint32_t)wave * 2048u, lda2, (uint32_t)kt * 64u,
+                                          2u * (uint32_t)s0.k, tid, i);
+        } else if constexpr (NN) {
+            const uint32_t lds = base + TILE * 4 + (uint32_t)(i - 2) * 1024u;
+            const uint32_t adv = (uint32_t)kt * (BK * 4u) * (uint32_t)s0.ldb;
+            // the ragged step's advance goes into the range-checked offset
+            if (full) dma16_s(rb, lds, offk[i - 2], adv);
+            else dma16(rb, lds, offk[i - 2] + adv);
+        } else {
+            if (full) dma_tile_full<BT, 256, 64, 2>(rb, base + TILE * 4, offb, (uint32_t)kt * 64u, i - 2);
+            else dma_tile<BT, 256, 64, 2>(rb, base + TILE * 4 - (uint32_t)wave * 2048u, ldb2, (uint32_t)kt * 64u,
+                                          2u * (uint32_t)s0.k, tid, i - 2);
+        }
+    };
+    // In step group u (8 k), lane l holds k 8 u + 4 h .. + 3 of its row of A
+    // and its column of B; MFMA p multiplies k 8 u + p and 8 u + 4 + p.
+    // The addresses within a stage are held for the whole loop and the stage is
+    // an offset of the instruction: VALU work takes MFMA time (see above).
+    f32x4 fa[2], fb[2];
+    const int sw = (rc >> 1) & 7;  // the rows' swizzle (wm, wn are multiples of 16)
+    const float *pa[4], *pb[NN ? 1 : 4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        pa[u] = sm + (wm + rc) * BK + 4 * ((2 * u + h) ^ sw);
+        if constexpr (!NN) pb[u] = sm + TILE + (wn + rc) * BK + 4 * ((2 * u + h) ^ sw);
+    }
+    if constexpr (NN) pb[0] = sm + TILE + 4 * h * BT + ((wn + rc) ^ (32 * h));
+    auto read = [&](int stage, int u, int slot) {
+        fa[slot] = *reinterpret_cast<const f32x4*>(pa[u] + stage * STAGE);
+        if constexpr (NN) {
+#pragma unroll
+            for (int p = 0; p < 4; ++p) fb[slot][p] = pb[0][stage * STAGE + (8 * u + p) * BT];
+        } else {
+            fb[slot] = *reinterpret_cast<const f32x4*>(pb[u] + stage * STAGE);
+        }
+    };
+    f32x16 tot, part;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) tot[q] = part[q] = 0.f;
+    auto step = [&](int kt, auto stage_tag) {
+        constexpr int U = decltype(stage_tag)::value;
+        if (kt + 2 < nk) wait_vmcnt<LOADS>();  // step kt + 2 may stay in flight
+        else wait_vmcnt<0>();
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            read(u < 3 ? U : (U + 1) & 3, (u + 1) & 3, (u + 1) & 1);
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                part = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[u & 1][p], fb[u & 1][p], part, 0, 0, 0);
+                if (u == 0) {  // one load behind each MFMA: a wave stalls while a load issues
+                    if (kt + 3 < nk) issue(kt + 3, (U + 3) & 3, p);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (kt == next_sum) {  // wave-uniform
+            next_sum += sum_steps;
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                tot[q] += part[q];
+                part[q] = 0.f;
+            }
+        }
+    };
+    for (int kt = 0; kt < 3 && kt < nk; ++kt)
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) issue(kt, kt, i);
+    if (nk > 2) wait_vmcnt<2 * LOADS>();
+    else wait_vmcnt<0>();
+    __syncthreads();
+    read(0, 0, 0);
+    for (int kt = 0; kt < nk; kt += 4) {
+        step(kt, std::integral_constant<int, 0>{});
+        if (kt + 1 >= nk) break;
+        step(kt + 1, std::integral_constant<int, 1>{});
+        if (kt + 2 >= nk) break;
+        step(kt + 2, std::integral_constant<int, 2>{});
+        if (kt + 3 >= nk) break;
+        step(kt + 3, std::integral_constant<int, 3>{});
+    }
+    tot += part;
+
+    for (int64_t k0 = 0; k0 < s1.k; k0 += 64) {
+        constexpr int LDX = 64 + 4;
+        float *xa = sm, *xb = sm + BT * LDX;
+        if (k0 > 0) load_ext(k0);
+        __syncthreads();  // the stages (the previous 64 columns) have been read
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int k = (int)lk + 4 * i + e;
+                const bool in = k0 + k < s1.k;  // a row's k past the segment are another row's
+                xa[lr * LDX + k] = in ? ea[i][e] : 0.f;
+                if constexpr (NN) xb[lr * LDX + k] = in ? eb[i][e] : 0.f;
+                else xb[(nc + 4 * i + e) * LDX + kr] = eb[i][e];
+            }
+        __syncthreads();
+        f32x16 ext;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) ext[q] = 0.f;
+        const int groups = (int)((s1.k - k0 < 64 ? s1.k - k0 : 64) + 7) / 8;
+        for (int u = 0; u < groups; ++u) {
+            const f32x4 a = *reinterpret_cast<const f32x4*>(&xa[(wm + rc) * LDX + 8 * u + 4 * h]);
+            const f32x4 b = *reinterpret_cast<const f32x4*>(&xb[(wn + rc) * LDX + 8 * u + 4 * h]);
+#pragma unroll
+            for (int p = 0; p < 4; ++p) ext = __builtin_amdgcn_mfma_f32_32x32x2f32(a[p], b[p], ext, 0, 0, 0);
+        }
+        tot += ext;
+    }
+    const int64_t n = n0 + wn + rc;
+    const float bv = (bias && n < N) ? bias[n] : 0.f;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        const int64_t m = m0 + wm + 8 * (q >> 2) + 4 * h + (q & 3);
+        if (m < M && n < N) C[m * ldc + n] = tot[q] + bv;
+    }
+}
+
 }  // namespace
 
 // GEMM args of columns [n0, n0 + n) of an output with BN-wide tiles (B rows,
@@ -943,6 +1152,31 @@ hipError_t launch_gemm_bf16_multi(int64_t M, const GemmOut* outs, int nout, hipS
     }
 }
 
+// Whether gemm_f32_tiled takes the product: its 64 x 64 tiles run in rounds of
+// one per CU (two resident tiles share the CU's MFMA rate), a step of 32 k in
+// 0.56 us, after about 6 us to fill the ring and add the rank-r columns;
+// gemm_f32_mfma's 32 x 32 tiles spread over any number of CUs and take
+// 0.82 ns each per step and 5 us. In units of the latter a round of steps costs
+// 683, the difference of the fixed parts 1200. Measured, 32 x 32 / this, us:
+// 2036x8960x1536 780 / 515, 2036x1536x8960 590 / 440, 1024x896x896 32 / 24,
+// 1024x1536x1536 61 / 57, 2036x1536x256 36 / 26; but 512x768x768 13.5 / 20,
+// 777x1536x1536 56 / 57, 106x8960x1536 52 / 57, 333x1536x8960 150 / 173.
+// It reads 16-byte chunks of the first segment's rows through 32-bit offsets.
+bool gemm_f32_large(int64_t M, int64_t N, bool nn, const GemmSegF32& s0, const GemmSegF32& s1, int cus) {
+    constexpr int64_t kLim = ((int64_t)1 << 31) - 256;
+    auto rows_fit = [&](int64_t ld, int64_t k) { return (63 * ld + k) * 4 < kLim; };
+    if (s0.k < 4 || s0.k % 4 != 0 || s0.lda % 4 != 0 || s0.ldb % 4 != 0) return false;
+    if ((reinterpret_cast<uintptr_t>(s0.a) | reinterpret_cast<uintptr_t>(s0.b)) & 15) return false;
+    if (!rows_fit(s0.lda, s0.k) || !rows_fit(s1.lda, s1.k)) return false;
+    if (nn ? (s0.k + 32) * s0.ldb * 4 >= kLim || !rows_fit(s1.ldb, s1.k)
+           : !rows_fit(s0.ldb, s0.k) || (s1.k + 64) * s1.ldb * 4 >= kLim)
+        return false;
+    const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64), tiles32 = ((M + 31) / 32) * ((N + 31) / 32);
+    if (tiles >= ((int64_t)1 << 31)) return false;
+    const double steps = (double)((s0.k + 31) / 32), rounds = (double)((tiles + cus - 1) / cus);
+    return 683.0 * rounds * steps + 1200.0 < (double)tiles32 * steps;
+}
+
 hipError_t launch_gemm_f32(bool nn, bool nn1, int64_t M, int64_t N, GemmSegF32 s0, GemmSegF32 s1, const float* bias,
                            float* c, int64_t ldc, hipStream_t stream) {
     const int64_t tiles_m = (M + 31) / 32, tiles_n = (N + 31) / 32;
@@ -960,6 +1194,13 @@ hipError_t launch_gemm_f32(bool nn, bool nn1, int64_t M, int64_t N, GemmSegF32 s
         return 32 * g.lda * 4 < kLim && (g_nn ? (g.k + 1) * g.ldb * 4 < kLim : 32 * g.ldb * 4 < kLim);
     };
     const bool buf = fits(s0, nn) && fits(s1, nn1);
+    if (nn != nn1 && gemm_f32_large(M, N, nn, s0, s1, cu_count())) {
+        const int tm = (int)((M + 63) / 64), tn64 = (int)((N + 63) / 64);
+        const dim3 g64((unsigned)(tm * tn64));
+        if (nn) gemm_f32_tiled<true><<<g64, 256, 0, stream>>>(M, N, a, b, bias, c, ldc, tm, tn64);
+        else gemm_f32_tiled<false><<<g64, 256, 0, stream>>>(M, N, a, b, bias, c, ldc, tm, tn64);
+        return hipGetLastError();
+    }
     auto go = [&](auto nn_tag, auto nn1_tag) {
         constexpr bool A = decltype(nn_tag)::value, B = decltype(nn1_tag)::value;
         if (buf) gemm_f32_mfma<A, B, true><<<grid, 256, 0, stream>>>(M, N, a, b, bias, c, ldc, tn);
