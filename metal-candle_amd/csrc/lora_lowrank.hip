@@ -29,6 +29,7 @@
 //
 // fp32 variants (plain FMA) serve act_dtype == MC_F32.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "lora_kernels.hpp"
@@ -1310,52 +1311,130 @@ __global__ __launch_bounds__(256) void lora_bwd_operands(OperandsBatch ob) {
 }
 
 // ------------------------------------------------------------ fp32 path
-// fp32 row projection: one workgroup per token t, ranks in chunks of 8. The
-// 256 threads take columns c = tid, tid + 256, ... of x's row (read once per
-// chunk, coalesced) and accumulate the chunk's 8 products per column in
-// column order; the 8 sums are reduced over each wave by butterfly and over
-// the 4 waves in wave order through LDS.
-__global__ __launch_bounds__(256) void rowproj_f32(const float* __restrict__ X, int64_t T, int64_t C,
-                                                   const float* __restrict__ P, int transpose_p, int r,
-                                                   float scale, const uint8_t* __restrict__ mask, float keep,
-                                                   float* __restrict__ out_t, float* __restrict__ out_ext,
-                                                   float ext_scale) {
-    const int64_t t = blockIdx.x;
-    const int lane = lane_id(), wave = threadIdx.x >> 6;
-    const float* xr = X + t * C;
-    __shared__ float red[4][8];
-    for (int j0 = 0; j0 < r; j0 += 8) {
-        const int nj = r - j0 < 8 ? r - j0 : 8;
-        float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        for (int64_t c = threadIdx.x; c < C; c += 256) {
-            const float xv = xr[c];
+// 16 bytes of a row that is 4-byte aligned only.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ f32x4 load4(const float* p) { return *reinterpret_cast<const f32x4u*>(p); }
+// The first n (<= 0: none) of 4 consecutive floats, zeros after them.
+__device__ __forceinline__ f32x4 load4_n(const float* p, int64_t n) {
+    f32x4 v;
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (j < nj) acc[j] += xv * (transpose_p ? P[c * r + j0 + j] : P[(int64_t)(j0 + j) * C + c]);
-        }
+    for (int e = 0; e < 4; ++e) v[e] = e < n ? p[e] : 0.f;
+    return v;
+}
+
+// Sum of the waves' values v(0) .. v(nw - 1): four at a time, in a fixed order.
+template <typename F>
+__device__ __forceinline__ float wave_tree(int nw, F&& v) {
+    float t = 0.f;
+    for (int w = 0; w < nw; w += 4) {
+        const float a = v(w) + (w + 1 < nw ? v(w + 1) : 0.f);
+        const float b = (w + 2 < nw ? v(w + 2) : 0.f) + (w + 3 < nw ? v(w + 3) : 0.f);
+        t = w == 0 ? a + b : t + (a + b);
+    }
+    return t;
+}
+
+// fp32 row projection v[t][j] = sum_c X[t][c] P(j, c) on v_mfma_f32_16x16x4_f32:
+// a workgroup owns 16 tokens and 16 RT ranks, its waves take every nw-th block
+// of 32 NB columns. Lane l supplies token (rank) l % 16 and, for MFMA q of a
+// 16-column group, column 4 (l / 16) + q, so a lane loads 16 bytes of its row
+// of x and four lanes a 64-byte segment; the next block is requested before a
+// block is multiplied. Bound by the reads of x: the one workgroup per token
+// that it replaces read all of P for each token (2036 x 8960, r 16: 280 -> 51
+// us; 2036 x 1536: 106 -> 12 us; 512 x 768, r 8: 10 -> 6.5 us).
+// Every 16 products are summed on their own, the 16s in pairs, these per wave
+// and then the waves in order.
+template <int RT> constexpr int kF32RowWaves = RT <= 2 ? 16 : 8;  // 128 or 256 registers per lane
+template <int RT> constexpr int kF32RowBlocks = RT == 1 ? 2 : 1;
+template <int RT, bool TP>
+__global__ __launch_bounds__(64 * kF32RowWaves<RT>) void rowproj_f32(const float* __restrict__ X, int64_t T,
+                                                                     int64_t C, const float* __restrict__ P, int r,
+                                                                     float scale, const uint8_t* __restrict__ mask,
+                                                                     float keep, float* __restrict__ out_t,
+                                                                     float* __restrict__ out_ext, float ext_scale) {
+    constexpr int NB = kF32RowBlocks<RT>, W = 32 * NB;
+    const int lane = lane_id(), wave = wave_id(), l16 = lane & 15, g = lane >> 4;
+    const int nw = (int)(blockDim.x >> 6);
+    const int64_t t0 = (int64_t)blockIdx.x * 16;
+    const int j0 = (int)blockIdx.y * 16 * RT;
+    const float* xr = X + (t0 + l16 < T ? t0 + l16 : T - 1) * C + 4 * g;  // rows past T are dropped below
+    struct Block {
+        f32x4 x[2 * NB], p[RT][2 * NB];
+    };
+    auto fetch = [&](int64_t c0, Block& f) {
+        const bool whole = c0 + W <= C;  // wave-uniform
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float v = wave_sum(acc[j]);
-            if (lane == 0) red[wave][j] = v;
+        for (int i = 0; i < 2 * NB; ++i) {
+            const int64_t c = c0 + 16 * i, left = C - c - 4 * g;
+            f.x[i] = whole ? load4(xr + c) : load4_n(xr + c, left);
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const int j = j0 + 16 * rt + l16, jc = j < r ? j : r - 1;
+                if constexpr (TP) {
+                    const float* pr = P + (c + 4 * g) * r + jc;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) f.p[rt][i][q] = whole || q < left ? pr[(int64_t)q * r] : 0.f;
+                } else {
+                    const float* pr = P + (int64_t)jc * C + c + 4 * g;
+                    f.p[rt][i] = whole ? load4(pr) : load4_n(pr, left);
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) f.p[rt][i][q] = j < r ? f.p[rt][i][q] : 0.f;
+            }
         }
-        __syncthreads();
-        if (threadIdx.x < nj) {
-            const int j = j0 + (int)threadIdx.x;
-            float v = red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
-            v *= scale;
-            if (mask) v = mask[t * r + j] ? v * keep : 0.f;
-            if (out_t) out_t[(int64_t)j * T + t] = v;
-            if (out_ext) out_ext[t * r + j] = v * ext_scale;
+    };
+    f32x4 tot[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) tot[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    Block cur, next;
+    int64_t c0 = W * (int64_t)wave;
+    if (c0 < C) fetch(c0, cur);
+    for (; c0 < C; c0 += W * nw) {
+        if (c0 + W * nw < C) fetch(c0 + W * nw, next);
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            f32x4 part[2 * NB];
+#pragma unroll
+            for (int i = 0; i < 2 * NB; ++i) {
+                part[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    part[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.x[i][q], cur.p[rt][i][q], part[i], 0, 0, 0);
+            }
+            if constexpr (NB == 2) tot[rt] += (part[0] + part[1]) + (part[2] + part[3]);
+            else tot[rt] += part[0] + part[1];
         }
-        __syncthreads();
+        cur = next;
+    }
+    // accumulator i of lane l is token 4 (l / 16) + i, rank l % 16
+    __shared__ float red[kF32RowWaves<RT>][RT][16][17];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) red[wave][rt][4 * g + i][l16] = tot[rt][i];
+    __syncthreads();
+    for (int o = (int)threadIdx.x; o < 256 * RT; o += (int)blockDim.x) {
+        const int rt = o >> 8, tl = o & 15, jl = (o >> 4) & 15, j = j0 + 16 * rt + jl;
+        const int64_t t = t0 + tl;
+        if (t >= T || j >= r) continue;
+        float v = scale * wave_tree(nw, [&](int w) { return red[w][rt][tl][jl]; });
+        if (mask) v = mask[t * r + j] ? v * keep : 0.f;
+        if (out_t) out_t[(int64_t)j * T + t] = v;
+        if (out_ext) out_ext[t * r + j] = v * ext_scale;
     }
 }
+
 // fp32 column reduction out[j][c] = scale * sum_t Pt[j][t] X[t][c] (or out
-// [c][j] with transpose_out): a workgroup owns 16 columns and a chunk of 8
-// ranks; its 256 threads are 4 column quads x 64 token slices, slice s
-// summing t = s, s + 64, ... in order (one 16-byte load of x per token when
-// C % 4 == 0, the 8 Pt values broadcast); the 64 slice sums are added in
-// slice order in two LDS stages (8 runs of 8, then the runs).
+// [c][j] with transpose_out) on v_mfma_f32_16x16x4_f32: a workgroup owns 64
+// columns and 16 RT ranks, its waves take every nw-th block of 16 tokens. Lane
+// l loads columns 4 (l % 16) .. + 3 of token 4 (l / 16) + q (whole 256-byte row
+// segments per 16 lanes), which are the operands of four 16-column tiles, tile
+// e holding columns 4 i + e, and 16 bytes of rank l % 16's row of Pt for the
+// four q. Bound by the reads of X, each rank group one pass over it: 2036
+// tokens, 1536 and 8960 columns, r 16: 53 -> 19 us against 8 ranks x 16
+// columns per workgroup on the vector unit. Every block's products are summed on
+// their own (in two chains of 8 where the registers allow it), the blocks per
+// wave and then the waves in order.
 // One or two reductions (dA over x and dB over dY) in one launch: blocks
 // [0, nblk0) take job 0, the rest job 1.
 struct ColF32Job {
@@ -1367,68 +1446,85 @@ struct ColF32Job {
     float* out;
     int64_t ctiles;
 };
-__global__ __launch_bounds__(256) void colreduce_f32(int64_t T, int r, ColF32Job ja, ColF32Job jb, int64_t nblk0) {
+template <int RT> constexpr int kF32ColWaves = RT == 1 ? 16 : 8;  // 128 or 256 registers per lane
+template <int RT>
+__global__ __launch_bounds__(64 * kF32ColWaves<RT>) void colreduce_f32(int64_t T, int r, ColF32Job ja, ColF32Job jb,
+                                                                    int64_t nblk0) {
     const bool second = (int64_t)blockIdx.x >= nblk0;  // workgroup-uniform
     const ColF32Job& J = second ? jb : ja;
     const int64_t b = (int64_t)blockIdx.x - (second ? nblk0 : 0);
     const float* __restrict__ X = J.X;
     const float* __restrict__ Pt = J.Pt;
     const int64_t C = J.C, ctiles = J.ctiles;
-    const int64_t c0 = (b % ctiles) * 16;
-    const int j0 = (int)(b / ctiles) * 8;
-    const int nj = r - j0 < 8 ? r - j0 : 8;
-    const int cq = threadIdx.x & 3, sl = threadIdx.x >> 2;
-    const int64_t c = c0 + 4 * cq;
-    const bool vec = (C & 3) == 0 && c + 3 < C;
-    float acc[8][4];
+    const int64_t c0 = (b % ctiles) * 64;
+    const int j0 = (int)(b / ctiles) * 16 * RT;
+    const int lane = lane_id(), wave = wave_id(), l16 = lane & 15, g = lane >> 4;
+    const int nw = (int)(blockDim.x >> 6);
+    const int64_t cleft = C - c0 - 4 * l16;
+    struct Block {
+        f32x4 x[4], a[RT];
+    };
+    auto fetch = [&](int64_t t0, Block& f) {
+        const int64_t tleft = T - t0 - 4 * g;
+        const bool whole = t0 + 16 <= T && c0 + 64 <= C;  // wave-uniform
+        const float* xr = X + (t0 + 4 * g) * C + c0 + 4 * l16;
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+        for (int q = 0; q < 4; ++q)
+            f.x[q] = whole ? load4(xr + (int64_t)q * C) : load4_n(xr + (int64_t)q * C, q < tleft ? cleft : 0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[j][e] = 0.f;
-    for (int64_t t = sl; t < T; t += 64) {
-        float xv[4];
-        if (vec) {
-            const float4 q = *reinterpret_cast<const float4*>(X + t * C + c);
-            xv[0] = q.x; xv[1] = q.y; xv[2] = q.z; xv[3] = q.w;
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) xv[e] = c + e < C ? X[t * C + c + e] : 0.f;
+        for (int rt = 0; rt < RT; ++rt) {
+            const int j = j0 + 16 * rt + l16;
+            const float* pr = Pt + (int64_t)(j < r ? j : r - 1) * T + t0 + 4 * g;
+            f.a[rt] = whole ? load4(pr) : load4_n(pr, tleft);
         }
+    };
+    constexpr int NC = RT == 1 ? 2 : 1;  // chains
+    f32x4 tot[RT][4];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float pv = j < nj ? Pt[(int64_t)(j0 + j) * T + t] : 0.f;
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[j][e] += pv * xv[e];
+        for (int e = 0; e < 4; ++e) tot[rt][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    Block cur, next;
+    int64_t t0 = 16 * (int64_t)wave;
+    if (t0 < T) fetch(t0, cur);
+    for (; t0 < T; t0 += 16 * nw) {
+        if (t0 + 16 * nw < T) fetch(t0 + 16 * nw, next);
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            f32x4 part[NC][4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    f32x4& p = part[q * NC / 4][e];
+                    const f32x4 c = q % (4 / NC) == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : p;
+                    p = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.a[rt][q], cur.x[q][e], c, 0, 0, 0);
+                }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) tot[rt][e] += NC == 2 ? part[0][e] + part[NC - 1][e] : part[0][e];
         }
+        cur = next;
     }
-    __shared__ float red[64][8][17];  // [slice][rank][column]
-    __shared__ float red2[8][8][17];  // [run][rank][column]
+    // accumulator i of tile e is rank 4 (l / 16) + i, column 4 (l % 16) + e;
+    // LDS rows of 68 floats keep both the 16-byte writes and the transposed
+    // reads off each other's banks
+    __shared__ __attribute__((aligned(16))) float red[kF32ColWaves<RT>][16][68];
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int rt = 0; rt < RT; ++rt) {
+        if (rt > 0) __syncthreads();
 #pragma unroll
-        for (int e = 0; e < 4; ++e) red[sl][j][4 * cq + e] = acc[j][e];
-    __syncthreads();
-    {
-        // thread -> (run, rank, 2 columns): 8 x 8 x 8 = 512 sums over 2 passes
-        for (int i = threadIdx.x; i < 8 * 8 * 16; i += 256) {
-            const int col = i & 15, j = (i >> 4) & 7, run = i >> 7;
-            float v = red[8 * run][j][col];
-#pragma unroll
-            for (int k = 1; k < 8; ++k) v += red[8 * run + k][j][col];
-            red2[run][j][col] = v;
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x < 8 * 16) {
-        const int col = threadIdx.x & 15, j = threadIdx.x >> 4;
-        float v = red2[0][j][col];
-#pragma unroll
-        for (int k = 1; k < 8; ++k) v += red2[k][j][col];
-        const int64_t cc = c0 + col;
-        if (j < nj && cc < C) {
-            v *= J.scale;
-            if (J.transpose_out) J.out[cc * r + j0 + j] = v;
-            else J.out[(int64_t)(j0 + j) * C + cc] = v;
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<f32x4*>(&red[wave][4 * g + i][4 * l16]) =
+                f32x4{tot[rt][0][i], tot[rt][1][i], tot[rt][2][i], tot[rt][3][i]};
+        __syncthreads();
+        for (int o = (int)threadIdx.x; o < 1024; o += (int)blockDim.x) {
+            const int jl = J.transpose_out ? o & 15 : o >> 6, cl = J.transpose_out ? o >> 4 : o & 63;
+            const int j = j0 + 16 * rt + jl;
+            const int64_t c = c0 + cl;
+            if (j >= r || c >= C) continue;
+            const float v = J.scale * wave_tree(nw, [&](int w) { return red[w][jl][cl]; });
+            if (J.transpose_out) J.out[c * r + j] = v;
+            else J.out[(int64_t)j * C + c] = v;
         }
     }
 }
@@ -1906,23 +2002,47 @@ hipError_t launch_rowproj_f32(const float* X, int64_t T, int64_t C, const float*
                               int r, float scale, const uint8_t* mask, float keep, float* out_t,
                               float* out_ext, float ext_scale, hipStream_t stream) {
     if (T >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
-    rowproj_f32<<<dim3((unsigned)T), 256, 0, stream>>>(X, T, C, P, transpose_p ? 1 : 0, r, scale, mask, keep, out_t,
-                                                       out_ext, ext_scale);
+    auto go = [&](auto rt_tag, auto tp_tag) {
+        constexpr int RT = decltype(rt_tag)::value;
+        constexpr bool TP = decltype(tp_tag)::value;
+        // a wave per block of columns, up to the waves the registers allow
+        constexpr int W = 32 * kF32RowBlocks<RT>;
+        const int nw = (int)std::min<int64_t>(kF32RowWaves<RT>, (C + W - 1) / W);
+        const dim3 grid((unsigned)((T + 15) / 16), (unsigned)((r + 16 * RT - 1) / (16 * RT)));
+        rowproj_f32<RT, TP><<<grid, 64 * nw, 0, stream>>>(X, T, C, P, r, scale, mask, keep, out_t, out_ext, ext_scale);
+    };
+    auto by_rank = [&](auto tp_tag) {
+        if (r <= 16) go(std::integral_constant<int, 1>{}, tp_tag);
+        else if (r <= 32) go(std::integral_constant<int, 2>{}, tp_tag);
+        else go(std::integral_constant<int, 4>{}, tp_tag);
+    };
+    if (transpose_p) by_rank(std::true_type{});
+    else by_rank(std::false_type{});
     return hipGetLastError();
 }
 
 hipError_t launch_colreduce_f32(const ColF32Call* calls, int n, int64_t T, int r, hipStream_t stream) {
     if (n < 1 || n > 2) return hipErrorInvalidValue;
+    const int rt = r <= 16 ? 1 : r <= 32 ? 2 : 4;
     ColF32Job j[2]{};
     int64_t nblk[2] = {0, 0};
     for (int i = 0; i < n; ++i) {
         const ColF32Call& c = calls[i];
-        j[i] = ColF32Job{c.X, c.C, c.Pt, c.scale, c.transpose_out ? 1 : 0, c.out, (c.C + 15) / 16};
-        nblk[i] = j[i].ctiles * ((r + 7) / 8);
+        j[i] = ColF32Job{c.X, c.C, c.Pt, c.scale, c.transpose_out ? 1 : 0, c.out, (c.C + 63) / 64};
+        nblk[i] = j[i].ctiles * ((r + 16 * rt - 1) / (16 * rt));
     }
     if (nblk[0] + nblk[1] >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
     if (nblk[0] + nblk[1] == 0) return hipSuccess;
-    colreduce_f32<<<dim3((unsigned)(nblk[0] + nblk[1])), 256, 0, stream>>>(T, r, j[0], n > 1 ? j[1] : j[0], nblk[0]);
+    const dim3 grid((unsigned)(nblk[0] + nblk[1]));
+    const ColF32Job& jb = n > 1 ? j[1] : j[0];
+    auto go = [&](auto rt_tag) {
+        constexpr int RT = decltype(rt_tag)::value;
+        const int nw = (int)std::min<int64_t>(kF32ColWaves<RT>, (T + 15) / 16);  // a wave per 16 tokens
+        colreduce_f32<RT><<<grid, 64 * nw, 0, stream>>>(T, r, j[0], jb, nblk[0]);
+    };
+    if (rt == 1) go(std::integral_constant<int, 1>{});
+    else if (rt == 2) go(std::integral_constant<int, 2>{});
+    else go(std::integral_constant<int, 4>{});
     return hipGetLastError();
 }
 

@@ -1,6 +1,7 @@
 """The float32 LoRA linear at the sizes where its kernels change: products of
 enough 64 x 64 tiles for the LDS-ring GEMM (ragged tiles, ragged last k steps,
-one to several 64-rank blocks) next to shapes that stay on the 32 x 32 one.
+one to several 64-rank blocks) next to shapes that stay on the 32 x 32 one, and
+the rank-r products at the edges of their tiles.
 
 Reference: the same composite in float64 on the GPU. Tolerance as in
 test_gpu_lora.py: max|out - ref| / max|ref| <= 1e-5.
@@ -58,6 +59,15 @@ def test_lora_f32_ring_gemm(mc, dev, T, K, N, r, p):
 def test_lora_f32_other_shapes(mc, dev, T, K, N, r):
     """Widths whose rows are not whole 16-byte chunks, and small products."""
     check_lora(mc, lora_case(dev, T, K, N, r, 0.0, T + K), 0.5, 0.0)
+
+
+@pytest.mark.parametrize("r", [1, 15, 16, 17, 32, 33, 64, 65, 129])
+@pytest.mark.parametrize("T,K,N", [(1, 5, 7), (17, 31, 33), (33, 64, 65), (250, 66, 127), (257, 1000, 130)])
+def test_lora_f32_rank_products(mc, dev, T, K, N, r):
+    """The rank-r products on the matrix cores: ranks around the 16-rank tiles
+    and 64-rank groups, tokens and columns around the 16-token and 32- / 64-
+    column blocks, rows that are not 16-byte aligned, dropout."""
+    check_lora(mc, lora_case(dev, T, K, N, r, 0.1, T + K + r), 2.0, 0.1)
 
 
 def test_lora_f32_ring_gemm_sees_only_its_rows(mc, dev):
