@@ -19,8 +19,11 @@
 // [4,28,4096,4096] score tensor has 1.9e9 elements. Longer rows (past 8
 // vectors per lane) take one workgroup per row with the row in the
 // registers of up to 1024 threads, and rows past that (128 KB) two
-// streaming passes; rows that are not whole 16-byte vectors take a scalar
-// kernel.
+// streaming passes. Rows that are not whole 16-byte vectors run on the same
+// one-wave kernels over the aligned vectors that cover them (RowVecs), or on a
+// scalar kernel past 8 vectors per lane.
+#include <type_traits>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -42,12 +45,74 @@ __device__ __forceinline__ int64_t row_limit(int64_t row, int64_t dim, int64_t c
     return causal_rows > 0 ? row % causal_rows + (dim - causal_rows) : dim - 1;
 }
 
+// The 16-byte vectors of one row. WHOLE: dim is a multiple of the vector, so
+// they are the row's own. Otherwise the row starts `lead` elements into the
+// first of the aligned vectors that cover it, and its first and last vector may
+// be shared with the neighbouring rows: their elements are loaded and masked
+// (index < 0 or past the row), and such a vector is stored element by element.
+// fp32 causal scores [4, 14, 777, 777], forward / backward: 100 / 87 us on the
+// scalar kernels (4 bytes per lane, a row read two or three times), 53 / 84 us
+// here from cold caches and 168 -> 94 us for the two in a loop; 776 columns
+// take 54 / 77 us.
+template <typename T, bool WHOLE> struct RowVecs {
+    static constexpr int N = BVec<T>::N, ES = (int)sizeof(T);
+    int lead, nvec, dim;
+    uint32_t bytes;  // from the first vector to the tensor's end (not WHOLE)
+    __device__ RowVecs(int64_t row, int64_t rows, int d) : dim(d) {
+        lead = WHOLE ? 0 : (int)(row * d % N);
+        nvec = WHOLE ? d / N : (lead + d + N - 1) / N;
+        const int64_t left = WHOLE ? 0 : ((rows - row) * d + lead) * ES;
+        bytes = left < 0x7fffffff ? (uint32_t)left : 0x7fffffffu;
+    }
+    __device__ int index(int vi, int e) const { return vi * N + e - lead; }
+    // element 0 of the vectors, from the tensor's start
+    __device__ int64_t first(int64_t row) const { return row * dim - lead; }
+    // Vector vi at byte offset base + 16 vi (ok: else zeros). The tensor's end
+    // may fall inside a vector: dwords past it load as zeros, and bf16 elements
+    // are read one by one there, as the last may be half of a dword.
+    __device__ void load(__amdgpu_buffer_rsrc_t r, uint32_t base, int vi, bool ok, float (&v)[N]) const {
+        const uint32_t off = ok ? base + (uint32_t)(vi * N * ES) : kOOB;
+        if constexpr (!WHOLE && ES == 2) {
+            const bool cut = ok && (uint32_t)(vi + 1) * 16u > bytes;
+            BVec<T>::load(r, cut ? kOOB : off, v);
+            if (__any(cut)) {
+#pragma unroll
+                for (int e = 0; e < N; ++e) {
+                    const uint16_t h = __builtin_amdgcn_raw_buffer_load_b16(r, (int)(cut ? off + 2u * e : kOOB), 0, 0);
+                    v[e] = cut ? bf16_to_f32(h) : v[e];
+                }
+            }
+        } else {
+            BVec<T>::load(r, off, v);
+        }
+    }
+    __device__ void store(__amdgpu_buffer_rsrc_t r, uint32_t base, int vi, const float (&o)[N]) const {
+        const uint32_t off = base + (uint32_t)(vi * N * ES);
+        const bool mine = vi < nvec;
+        const bool full = mine && (WHOLE || (index(vi, 0) >= 0 && index(vi, N - 1) < dim));
+        BVec<T>::store_nt(r, full ? off : kOOB, o);
+        if constexpr (!WHOLE) {
+            const bool part = mine && !full;
+            if (__any(part)) {
+#pragma unroll
+                for (int e = 0; e < N; ++e) {
+                    const uint32_t at = part && index(vi, e) >= 0 && index(vi, e) < dim ? off + (uint32_t)(e * ES) : kOOB;
+                    if constexpr (ES == 4)
+                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[e]), r, (int)at, 0, 0);
+                    else
+                        __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16(o[e]), r, (int)at, 0, 0);
+                }
+            }
+        }
+    }
+};
+
 // Vector path: the 4 rows of a workgroup through one buffer resource (a
-// wave's row at a scalar byte offset); every load of the row is issued
-// before any use, with wholly masked vectors and vectors past the row given
-// out-of-range offsets (no memory traffic, zeros), and the masks applied as
-// value selects.
-template <typename T, int VPL>
+// wave's row at a scalar byte offset; not WHOLE: a resource per wave); every
+// load of the row is issued before any use, with wholly masked vectors and
+// vectors past the row given out-of-range offsets (no memory traffic, zeros),
+// and the masks applied as value selects.
+template <typename T, int VPL, bool WHOLE>
 __global__ __launch_bounds__(256) void softmax_fwd_vec(int64_t rbase, int64_t rows, int dim, int64_t causal_rows,
                                                        const T* __restrict__ s, T* __restrict__ p) {
     constexpr int N = BVec<T>::N;
@@ -57,18 +122,18 @@ __global__ __launch_bounds__(256) void softmax_fwd_vec(int64_t rbase, int64_t ro
     const int64_t r0 = rbase + (int64_t)blockIdx.x * kRowsPerBlock;
     const int64_t row = r0 + wave;
     if (row >= rows) return;
+    const RowVecs<T, WHOLE> rv(row, rows, dim);
     const int64_t nrows = rows - r0 < kRowsPerBlock ? rows - r0 : kRowsPerBlock;
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(s + r0 * dim, nrows * dim * ES);
-    const __amdgpu_buffer_rsrc_t rp = make_rsrc(p + r0 * dim, nrows * dim * ES);
-    const int nvec = dim / N;
+    const int64_t at = WHOLE ? r0 * dim : rv.first(row), bytes = WHOLE ? nrows * dim * ES : (int64_t)rv.bytes;
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(s + at, bytes);
+    const __amdgpu_buffer_rsrc_t rp = make_rsrc(p + at, bytes);
     const int lim = (int)row_limit(row, dim, causal_rows);
-    const uint32_t rowoff = (uint32_t)(wave * dim * ES);
+    const uint32_t rowoff = WHOLE ? (uint32_t)(wave * dim * ES) : 0u;
     float v[VPL][N];
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
         const int vi = lane + i * kWave;
-        const bool ok = vi < nvec && vi * N <= lim;
-        BVec<T>::load(rs, ok ? rowoff + (uint32_t)(vi * N * ES) : kOOB, v[i]);
+        rv.load(rs, rowoff, vi, vi < rv.nvec && rv.index(vi, 0) <= lim, v[i]);
     }
     float m = -INFINITY;
 #pragma unroll
@@ -76,7 +141,8 @@ __global__ __launch_bounds__(256) void softmax_fwd_vec(int64_t rbase, int64_t ro
         const int vi = lane + i * kWave;
 #pragma unroll
         for (int e = 0; e < N; ++e) {
-            const bool valid = vi < nvec && vi * N + e <= lim;
+            const int j = rv.index(vi, e);
+            const bool valid = vi < rv.nvec && j <= lim && (WHOLE || j >= 0);
             v[i][e] = valid ? v[i][e] : -INFINITY;
             m = fmaxf(m, v[i][e]);
         }
@@ -95,11 +161,14 @@ __global__ __launch_bounds__(256) void softmax_fwd_vec(int64_t rbase, int64_t ro
     const float inv = 1.0f / sum;
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
-        const int vi = lane + i * kWave;
         float o[N];
 #pragma unroll
-        for (int e = 0; e < N; ++e) o[e] = v[i][e] * inv;
-        BVec<T>::store_nt(rp, vi < nvec ? rowoff + (uint32_t)(vi * N * ES) : kOOB, o);
+        for (int e = 0; e < N; ++e) {
+            o[e] = v[i][e] * inv;
+            // masked columns of a row without a finite maximum are zeros here, as in the scalar form
+            if constexpr (!WHOLE) o[e] = rv.index(lane + i * kWave, e) <= lim ? o[e] : 0.f;
+        }
+        rv.store(rp, rowoff, lane + i * kWave, o);
     }
 }
 
@@ -125,7 +194,7 @@ __global__ __launch_bounds__(256) void softmax_fwd_scalar(int64_t rbase, int64_t
     }
 }
 
-template <typename T, int VPL>
+template <typename T, int VPL, bool WHOLE>
 __global__ __launch_bounds__(64 * kBwdRowsPerBlock) void softmax_bwd_vec(int64_t rbase, int64_t rows, int dim,
                                                                           int64_t causal_rows,
                                                                           const T* __restrict__ p,
@@ -138,20 +207,21 @@ __global__ __launch_bounds__(64 * kBwdRowsPerBlock) void softmax_bwd_vec(int64_t
     const int64_t r0 = rbase + (int64_t)blockIdx.x * kBwdRowsPerBlock;
     const int64_t row = r0 + wave;
     if (row >= rows) return;
+    const RowVecs<T, WHOLE> rv(row, rows, dim);
     const int64_t nrows = rows - r0 < kBwdRowsPerBlock ? rows - r0 : kBwdRowsPerBlock;
-    const __amdgpu_buffer_rsrc_t rp = make_rsrc(p + r0 * dim, nrows * dim * ES);
-    const __amdgpu_buffer_rsrc_t rg = make_rsrc(dp + r0 * dim, nrows * dim * ES);
-    const __amdgpu_buffer_rsrc_t rd = make_rsrc(ds + r0 * dim, nrows * dim * ES);
-    const int nvec = dim / N;
+    const int64_t at = WHOLE ? r0 * dim : rv.first(row), bytes = WHOLE ? nrows * dim * ES : (int64_t)rv.bytes;
+    const __amdgpu_buffer_rsrc_t rp = make_rsrc(p + at, bytes);
+    const __amdgpu_buffer_rsrc_t rg = make_rsrc(dp + at, bytes);
+    const __amdgpu_buffer_rsrc_t rd = make_rsrc(ds + at, bytes);
     const int lim = (int)row_limit(row, dim, causal_rows);
-    const uint32_t rowoff = (uint32_t)(wave * dim * ES);
+    const uint32_t rowoff = WHOLE ? (uint32_t)(wave * dim * ES) : 0u;
     float pv[VPL][N], gv[VPL][N];
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
         const int vi = lane + i * kWave;
-        const uint32_t off = (vi < nvec && vi * N <= lim) ? rowoff + (uint32_t)(vi * N * ES) : kOOB;
-        BVec<T>::load(rp, off, pv[i]);
-        BVec<T>::load(rg, off, gv[i]);
+        const bool ok = vi < rv.nvec && rv.index(vi, 0) <= lim;
+        rv.load(rp, rowoff, vi, ok, pv[i]);
+        rv.load(rg, rowoff, vi, ok, gv[i]);
     }
     float dot = 0.f;
 #pragma unroll
@@ -160,18 +230,24 @@ __global__ __launch_bounds__(64 * kBwdRowsPerBlock) void softmax_bwd_vec(int64_t
 #pragma unroll
         for (int e = 0; e < N; ++e) {
             // masked: p = 0 by definition (and dp is not read there)
-            pv[i][e] = (vi < nvec && vi * N + e <= lim) ? pv[i][e] : 0.f;
+            const int j = rv.index(vi, e);
+            const bool valid = vi < rv.nvec && j <= lim && (WHOLE || j >= 0);
+            pv[i][e] = valid ? pv[i][e] : 0.f;
+            if constexpr (!WHOLE) gv[i][e] = valid ? gv[i][e] : 0.f;  // a neighbour's may be anything
             dot += pv[i][e] * gv[i][e];
         }
     }
     dot = wave_sum(dot);
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
-        const int vi = lane + i * kWave;
         float o[N];
 #pragma unroll
-        for (int e = 0; e < N; ++e) o[e] = pv[i][e] * (gv[i][e] - dot);
-        BVec<T>::store_nt(rd, vi < nvec ? rowoff + (uint32_t)(vi * N * ES) : kOOB, o);
+        for (int e = 0; e < N; ++e) {
+            o[e] = pv[i][e] * (gv[i][e] - dot);
+            // past the causal limit the scalar form writes zeros whatever the row's dot is
+            if constexpr (!WHOLE) o[e] = rv.index(lane + i * kWave, e) <= lim ? o[e] : 0.f;
+        }
+        rv.store(rd, rowoff, lane + i * kWave, o);
     }
 }
 
@@ -432,19 +508,26 @@ __global__ __launch_bounds__(kWideThreads) void softmax_bwd_stream(int64_t row0,
     }
 }
 
-// Row paths by length (rows of 16-byte vectors; ragged rows take the scalar
-// kernels): one wave per row up to 8 vectors per lane, a workgroup per row
+// Row paths by length: one wave per row up to 8 vectors per lane (kWaveShared:
+// rows that are not whole 16-byte vectors, over the aligned vectors that cover
+// them; longer ones take the scalar kernels), a workgroup per row
 // up to max_vpl vectors per thread of 1024 threads, else two streaming
 // passes. (One wave at 9-16 vectors per lane measured slower than the
 // workgroup per row: bf16 [8192, 8192] backward 137 against 61 us, forward
 // 48 against 44 us.) The bf16 backward holds at most 4 vectors of p and 4 of dp per
 // thread: at 8 it needs more than the 128 registers a 1024-thread workgroup
 // leaves each thread.
-enum class RowPath { kScalar, kWave, kWide, kStream };
+enum class RowPath { kScalar, kWave, kWaveShared, kWide, kStream };
+
+// Most vectors a row of dim elements covers, wherever it starts.
+template <typename T>
+int64_t row_vectors(int64_t dim) {
+    return dim % Vec16<T>::N == 0 ? dim / Vec16<T>::N : (dim + 2 * (Vec16<T>::N - 1)) / Vec16<T>::N;
+}
 
 template <typename T>
 RowPath row_path(int64_t dim, int max_vpl) {
-    if (dim % Vec16<T>::N != 0) return RowPath::kScalar;
+    if (dim % Vec16<T>::N != 0) return row_vectors<T>(dim) <= 8 * kWave ? RowPath::kWaveShared : RowPath::kScalar;
     const int64_t nvec = dim / Vec16<T>::N;
     if (nvec <= 8 * kWave) return RowPath::kWave;
     if (nvec <= (int64_t)max_vpl * kWideThreads) return RowPath::kWide;
@@ -475,11 +558,14 @@ void for_row_chunks(int64_t rows, int threads, F&& launch, int rows_per_block = 
     }
 }
 
-template <typename T>
-int vpl_for(int64_t dim) {
-    const int64_t nvec = dim / Vec16<T>::N;
-    const int64_t per = (nvec + kWave - 1) / kWave;
-    return per <= 1 ? 1 : per <= 2 ? 2 : per <= 4 ? 4 : 8;
+// go(std::integral_constant<int, vectors per lane of the one-wave kernels>)
+template <typename T, typename F>
+void by_vpl(int64_t dim, F&& go) {
+    const int64_t per = (row_vectors<T>(dim) + kWave - 1) / kWave;
+    if (per <= 1) go(std::integral_constant<int, 1>{});
+    else if (per <= 2) go(std::integral_constant<int, 2>{});
+    else if (per <= 4) go(std::integral_constant<int, 4>{});
+    else go(std::integral_constant<int, 8>{});
 }
 
 template <typename T>
@@ -501,17 +587,17 @@ hipError_t fwd_impl(int64_t rows, int64_t dim, int64_t causal, const void* s, vo
         for_row_chunks(rows, kWideThreads, [&](int64_t r0, dim3 g) {
             softmax_fwd_stream<T><<<g, kWideThreads, 0, st>>>(r0, dim, causal, sp, pp);
         });
-    } else if (path == RowPath::kWave) {
+    } else if (path == RowPath::kWave || path == RowPath::kWaveShared) {
         const int d = (int)dim;
-        const int vpl = vpl_for<T>(dim);
-        for_row_chunks(rows, 256, [&](int64_t r0, dim3 g) {
-            switch (vpl) {
-                case 1: softmax_fwd_vec<T, 1><<<g, 256, 0, st>>>(r0, rows, d, causal, sp, pp); break;
-                case 2: softmax_fwd_vec<T, 2><<<g, 256, 0, st>>>(r0, rows, d, causal, sp, pp); break;
-                case 4: softmax_fwd_vec<T, 4><<<g, 256, 0, st>>>(r0, rows, d, causal, sp, pp); break;
-                default: softmax_fwd_vec<T, 8><<<g, 256, 0, st>>>(r0, rows, d, causal, sp, pp); break;
-            }
-        }, kRowsPerBlock);
+        const bool whole = path == RowPath::kWave;
+        auto go = [&](auto vpl_tag) {
+            constexpr int VPL = decltype(vpl_tag)::value;
+            for_row_chunks(rows, 256, [&](int64_t r0, dim3 g) {
+                if (whole) softmax_fwd_vec<T, VPL, true><<<g, 256, 0, st>>>(r0, rows, d, causal, sp, pp);
+                else softmax_fwd_vec<T, VPL, false><<<g, 256, 0, st>>>(r0, rows, d, causal, sp, pp);
+            }, kRowsPerBlock);
+        };
+        by_vpl<T>(dim, go);
     } else {
         for_row_chunks(rows, 256, [&](int64_t r0, dim3 g) {
             softmax_fwd_scalar<T><<<g, 256, 0, st>>>(r0, rows, dim, causal, sp, pp);
@@ -544,18 +630,18 @@ hipError_t bwd_impl(int64_t rows, int64_t dim, int64_t causal, const void* p, co
         for_row_chunks(rows, kWideThreads, [&](int64_t r0, dim3 g) {
             softmax_bwd_stream<T><<<g, kWideThreads, 0, st>>>(r0, dim, causal, pp, gp, dsp);
         });
-    } else if (path == RowPath::kWave) {
+    } else if (path == RowPath::kWave || path == RowPath::kWaveShared) {
         const int d = (int)dim;
-        const int vpl = vpl_for<T>(dim);
+        const bool whole = path == RowPath::kWave;
         constexpr int nt = 64 * kBwdRowsPerBlock;
-        for_row_chunks(rows, nt, [&](int64_t r0, dim3 g) {
-            switch (vpl) {
-                case 1: softmax_bwd_vec<T, 1><<<g, nt, 0, st>>>(r0, rows, d, causal, pp, gp, dsp); break;
-                case 2: softmax_bwd_vec<T, 2><<<g, nt, 0, st>>>(r0, rows, d, causal, pp, gp, dsp); break;
-                case 4: softmax_bwd_vec<T, 4><<<g, nt, 0, st>>>(r0, rows, d, causal, pp, gp, dsp); break;
-                default: softmax_bwd_vec<T, 8><<<g, nt, 0, st>>>(r0, rows, d, causal, pp, gp, dsp); break;
-            }
-        }, kBwdRowsPerBlock);
+        auto go = [&](auto vpl_tag) {
+            constexpr int VPL = decltype(vpl_tag)::value;
+            for_row_chunks(rows, nt, [&](int64_t r0, dim3 g) {
+                if (whole) softmax_bwd_vec<T, VPL, true><<<g, nt, 0, st>>>(r0, rows, d, causal, pp, gp, dsp);
+                else softmax_bwd_vec<T, VPL, false><<<g, nt, 0, st>>>(r0, rows, d, causal, pp, gp, dsp);
+            }, kBwdRowsPerBlock);
+        };
+        by_vpl<T>(dim, go);
     } else {
         for_row_chunks(rows, 256, [&](int64_t r0, dim3 g) {
             softmax_bwd_scalar<T><<<g, 256, 0, st>>>(r0, rows, dim, causal, pp, gp, dsp);
