@@ -70,6 +70,7 @@ struct LoraGroupFwdWs {
     size_t bt_ext[kLoraMaxProj];   // per projection: bf16 [N_g][rext]
     size_t hs_ext;                 // bf16 [T][G rext]: s Hd of every projection
     size_t part;                   // split row projection: f32 [passes][splits][T][16 rc] partials of H
+    size_t small;                  // few tokens: the partial sums of H (lora_small_ws)
     size_t total;
 };
 struct LoraGroupBwdWs {
@@ -95,6 +96,13 @@ hipError_t launch_lora_group_fwd(const mc_lora_desc& d, const void* x, const Lor
 hipError_t launch_lora_group_bwd(const mc_lora_desc& d, const void* x, const LoraProj* proj, int count,
                                  const float* const* h_save, const void* const* dY, void* dX, float* const* dA,
                                  float* const* dB, void* ws, hipStream_t stream);
+
+// The grouped forward of a few tokens (lora_small.hip), with its own partial
+// sums in ws (lora_small_ws bytes).
+constexpr int kSmallTokens = 32, kSmallRanks = 64;
+size_t lora_small_ws(int64_t T, int64_t K, int r, int count);
+hipError_t launch_lora_small_fwd(const mc_lora_desc& d, const void* x, const LoraProj* proj, int count, void* const* y,
+                                 float* const* h_save, void* ws, hipStream_t stream);
 
 // out [cols][rows] = in [rows][cols]^T, bf16
 hipError_t launch_transpose_bf16(const void* in, int64_t rows, int64_t cols, void* out, hipStream_t stream);

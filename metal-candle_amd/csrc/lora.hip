@@ -122,6 +122,11 @@ bool bwd_rowsplit(const Dims& m, const int64_t* N, int count) {
 // operand path, whose per-step operand split is the kernel's bottleneck.
 bool bwd_colsplit(const Dims& m, const int64_t* N, int count) { return bwd_rowsplit(m, N, count) && m.T % 8 == 0; }
 
+// Few tokens take two launches that read W row by row instead of the tiled
+// path's three. A rule on the tokens and ranks only, so a grouped call still
+// computes the sums of single calls.
+bool fwd_small(const Dims& m) { return m.bf16 && m.T <= kSmallTokens && m.r <= kSmallRanks; }
+
 // bf16 projections whose K or N is not a multiple of 8 (rows not made of
 // 16-byte chunks) run on copies zero-padded to multiples of 8: a padded
 // feature adds exact zeros to every product, so y, dX, dA and dB are the
@@ -312,6 +317,8 @@ LoraGroupFwdWs lora_group_fwd_ws(const mc_lora_desc& d, const int64_t* N, int co
         const int ld = rowsplit_ld((count < ppp ? count : ppp) * m.r);
         off += align256((size_t)npass * rowsplit_splits(m.T, m.K) * m.T * ld * 4);
     }
+    w.small = off;
+    if (fwd_small(m)) off += align256(lora_small_ws(m.T, m.K, m.r, count));
     w.total = off;
     return w;
 }
@@ -470,6 +477,12 @@ hipError_t launch_lora_group_fwd(const mc_lora_desc& d, const void* x, const Lor
     const LoraGroupFwdWs w = lora_group_fwd_ws(d, Ns, count);
     char* base = static_cast<char*>(ws);
     const uint16_t* xb = static_cast<const uint16_t*>(x);
+    if (fwd_small(m)) {
+        int64_t sumN = 0;
+        for (int g = 0; g < count; ++g) sumN += Ns[g];
+        auto sc = gemm_scope(st, m.T, sumN, m.K, m.r, m.r, 2);
+        return launch_lora_small_fwd(d, x, proj, count, y, h_save, base + w.small, st);
+    }
     uint16_t* hs = reinterpret_cast<uint16_t*>(base + w.hs_ext);
     const int ext_ld = count * m.rext;
     const int ppp = proj_per_pass(m.r);
