@@ -15,8 +15,8 @@
 // waves, each a WM x WN block of MFMA 32x32x16 bf16 tiles with fp32
 // accumulators. The tiles are chosen per shape (choose_gemm_plan): 256 x 256,
 // 256 x 192 or 256 x 128 with 8 waves and one workgroup per CU for the
-// large layer products, 128 x 128 with 4 waves where there are too few large
-// tiles to fill the 256 CUs; or 256 x 256 tiles over most columns and a
+// large layer products, 128 x 128 or 64 x 64 with 4 waves where there are too
+// few large tiles to fill the 256 CUs; or 256 x 256 tiles over most columns and a
 // narrower shape over the rest in one launch (gemm_bf16_split), so that the
 // widest tile fills whole rounds of CUs.
 //  - Operands go straight from HBM/L2 into LDS with buffer_load ... lds
@@ -989,8 +989,59 @@ double tile_speed(GemmTile t, int64_t K) {
 }
 
 void tile_dims(GemmTile t, int& bm, int& bn) {
-    bm = t == GemmTile::k128x128 ? 128 : 256;
-    bn = t == GemmTile::k256x256 ? 256 : t == GemmTile::k256x192 ? 192 : 128;
+    switch (t) {
+        case GemmTile::k256x256: bm = 256; bn = 256; break;
+        case GemmTile::k256x192: bm = 256; bn = 192; break;
+        case GemmTile::k256x128: bm = 256; bn = 128; break;
+        case GemmTile::k64x64: bm = 64; bn = 64; break;
+        default: bm = 128; bn = 128; break;
+    }
+}
+
+int64_t tile_count(GemmTile t, int64_t M, const int64_t* Ns, int nout) {
+    int bm, bn;
+    tile_dims(t, bm, bn);
+    int64_t cols = 0;
+    for (int o = 0; o < nout; ++o) cols += (Ns[o] + bn - 1) / bn;
+    return (M + bm - 1) / bm * cols;
+}
+
+// Time in us of `tiles` tiles of one shape and K columns when they are few
+// rounds, measured per step of 64 columns with 32 to 256 CUs busy (a small
+// tile's step is bound by its latency, not by its area, which is why the area
+// ratios of tile_speed do not hold here), plus the first loads and the epilogue.
+double few_rounds_us(GemmTile t, int64_t tiles, int64_t K, int cus) {
+    const double nk = (double)((K + 63) / 64), rounds = (double)((tiles + cus - 1) / cus);
+    switch (t) {
+        case GemmTile::k256x256: return rounds * 1.12 * nk + 4.0;
+        case GemmTile::k256x192: return rounds * 0.95 * nk + 4.0;
+        case GemmTile::k256x128: return rounds * 0.78 * nk + 4.0;
+        case GemmTile::k128x128: return rounds * 0.54 * nk + 4.0;
+        // two (64 x 64: up to two) workgroups of a CU at a time
+        case GemmTile::k128x128Pair: return (double)((tiles + 2 * cus - 1) / (2 * cus)) * 0.92 * nk + 4.0;
+        default: return (tiles <= cus ? 0.33 : 0.42 * (double)((tiles + 2 * cus - 1) / (2 * cus))) * nk + 3.5;
+    }
+}
+
+// Where the shape that the full-round estimate picked runs in at most two
+// rounds, a small grid: 64 x 64 tiles, or two 128 x 128 workgroups per CU, if
+// they are estimated at least 5% faster. All shapes add a product's columns in
+// the same order, so the choice changes no result. Measured, before / after,
+// us, M x N x K: 777x8960x1536 37 / 27.5, 300x18944x3584 67 / 52 (pairs);
+// 777x1536x8960 75 / 61, 100x3584x18944 156 / 98, 1243x512x3584 33 / 22,
+// 463x256x1536 16.7 / 11.2, 8192x128x896 11.7 / 8.5 (64 x 64).
+GemmTile small_grid_tile(GemmTile picked, int64_t M, const int64_t* Ns, int nout, int64_t K, int cus) {
+    const int64_t n = tile_count(picked, M, Ns, nout);
+    if (n > 2 * (int64_t)cus) return picked;
+    GemmTile best = picked;
+    double best_us = 0.95 * few_rounds_us(picked, n, K, cus);
+    for (GemmTile t : {GemmTile::k128x128Pair, GemmTile::k64x64}) {
+        const int64_t m = tile_count(t, M, Ns, nout);
+        if (t == GemmTile::k64x64 && m > 2 * (int64_t)cus) continue;
+        const double e = few_rounds_us(t, m, K, cus);
+        if (e < best_us) { best_us = e; best = t; }
+    }
+    return best;
 }
 
 // Estimated time of n1 tiles of duration t1 followed by n2 tiles of
@@ -1032,7 +1083,8 @@ double plan_time_multi(int64_t M, const int64_t* Ns, int nout, int64_t K, GemmTi
     return list_time(((M + bm - 1) / bm) * cols, (double)bm * bn / tile_speed(t, K), 0, 0.0, cus);
 }
 
-GemmPlan choose_gemm_plan(int64_t M, int64_t N, int64_t K, int cus) {
+// The plan by the full-round estimate.
+GemmPlan choose_round_plan(int64_t M, int64_t N, int64_t K, int cus) {
     // One tile shape over all of N, or 256 x 256 tiles over the first n1 =
     // 256 j columns and a narrower shape over the rest, whichever list_time
     // estimates fastest. The split lets the wide tile fill whole rounds
@@ -1065,6 +1117,13 @@ GemmPlan choose_gemm_plan(int64_t M, int64_t N, int64_t K, int cus) {
     return best;
 }
 
+GemmPlan choose_gemm_plan(int64_t M, int64_t N, int64_t K, int cus) {
+    const GemmPlan p = choose_round_plan(M, N, K, cus);
+    if (p.n1 < N) return p;
+    const GemmTile t = small_grid_tile(p.main, M, &N, 1, K, cus);
+    return GemmPlan{t, t, N};
+}
+
 hipError_t launch_gemm_bf16(int64_t M, int64_t N, const GemmSeg* segs, int nseg, const uint16_t* bias, uint16_t* c,
                             int64_t ldc, hipStream_t stream) {
     int64_t K = 0;
@@ -1084,6 +1143,10 @@ hipError_t launch_gemm_bf16(int64_t M, int64_t N, const GemmSeg* segs, int nseg,
             return launch_cfg<256, 192, 64, 96, 64, 2>(M, N, segs, nseg, bias, c, ldc, stream, 4);
         case GemmTile::k256x128:  // 8 waves of 64 x 64, 3 stages (144 KB LDS)
             return launch_cfg<256, 128, 64, 64, 64, 3>(M, N, segs, nseg, bias, c, ldc, stream, 4);
+        case GemmTile::k128x128Pair:  // 4 waves of 64 x 64, 2 stages (64 KB LDS: two workgroups per CU)
+            return launch_cfg<128, 128, 64, 64, 64, 2>(M, N, segs, nseg, bias, c, ldc, stream, 4);
+        case GemmTile::k64x64:    // 4 waves of 32 x 32, 4 stages (64 KB LDS)
+            return launch_cfg<64, 64, 32, 32, 64, 4>(M, N, segs, nseg, bias, c, ldc, stream, 4);
         default:                  // 4 waves of 64 x 64, 3 stages (96 KB LDS)
             return launch_cfg<128, 128, 64, 64, 64, 3>(M, N, segs, nseg, bias, c, ldc, stream, 4);
     }
@@ -1126,7 +1189,7 @@ bool gemm_bf16_multi_one_launch(int64_t M, const GemmOut* outs, int nout) {
     const int cus = cu_count();
     const GemmTile t = choose_multi_tile(M, Ns, nout, K, cus);
     double sep = 0.0;
-    for (int o = 0; o < nout; ++o) sep += plan_time(M, Ns[o], K, choose_gemm_plan(M, Ns[o], K, cus), cus);
+    for (int o = 0; o < nout; ++o) sep += plan_time(M, Ns[o], K, choose_round_plan(M, Ns[o], K, cus), cus);
     return !(sep < plan_time_multi(M, Ns, nout, K, t, cus));
 }
 
@@ -1143,11 +1206,14 @@ hipError_t launch_gemm_bf16_multi(int64_t M, const GemmOut* outs, int nout, hipS
     int64_t K = 0;
     for (int o = 0; o < nout; ++o) Ns[o] = outs[o].N;
     for (int i = 0; i < outs[0].nseg; ++i) K += outs[0].seg[i].k;
-    const GemmTile t = choose_multi_tile(M, Ns, nout, K, cu_count());
+    const int cus = cu_count();
+    const GemmTile t = small_grid_tile(choose_multi_tile(M, Ns, nout, K, cus), M, Ns, nout, K, cus);
     switch (t) {
         case GemmTile::k256x256: return launch_multi<256, 256, 128, 64, 64, 2>(M, outs, nout, stream, 4);
         case GemmTile::k256x192: return launch_multi<256, 192, 64, 96, 64, 2>(M, outs, nout, stream, 4);
         case GemmTile::k256x128: return launch_multi<256, 128, 64, 64, 64, 3>(M, outs, nout, stream, 4);
+        case GemmTile::k128x128Pair: return launch_multi<128, 128, 64, 64, 64, 2>(M, outs, nout, stream, 4);
+        case GemmTile::k64x64: return launch_multi<64, 64, 32, 32, 64, 4>(M, outs, nout, stream, 4);
         default: return launch_multi<128, 128, 64, 64, 64, 3>(M, outs, nout, stream, 4);
     }
 }

@@ -273,8 +273,10 @@ hipError_t launch_gemm_bf16_multi(int64_t M, const GemmOut* outs, int nout, hipS
 bool gemm_bf16_multi_one_launch(int64_t M, const GemmOut* outs, int nout);
 // Workgroup tiles of the bf16 GEMM for an M x N output with reduction length
 // K on `cus` compute units: `main` over columns [0, n1), `tail` over [n1, N)
-// (n1 == N: one tile shape; otherwise main is 256 x 256).
-enum class GemmTile { k256x256, k256x192, k256x128, k128x128 };
+// (n1 == N: one tile shape; otherwise main is 256 x 256). k128x128Pair is the
+// 128 x 128 tile with two stages instead of three, so that two workgroups share
+// a CU; k64x64 is for grids too small for 128 x 128 tiles to fill the CUs.
+enum class GemmTile { k256x256, k256x192, k256x128, k128x128, k128x128Pair, k64x64 };
 struct GemmPlan {
     GemmTile main, tail;
     int64_t n1;
