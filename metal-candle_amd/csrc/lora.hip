@@ -127,6 +127,19 @@ bool bwd_colsplit(const Dims& m, const int64_t* N, int count) { return bwd_rowsp
 // computes the sums of single calls.
 bool fwd_small(const Dims& m) { return m.bf16 && m.T <= kSmallTokens && m.r <= kSmallRanks; }
 
+// The forward's preparation and row projection as one launch
+// (launch_lora_fwd_operands). It reads x once per projection and repeats A's
+// strided reads for every 16 tokens, so it wins while launches and the wait
+// between them are the larger part. Forward, two launches -> one: K 1536,
+// N 8960, T 777 40.7 -> 34.5 us; K 3584, N 512, T 1243 42.5 -> 33.2; K 1536,
+// N 256, T 2048 23.7 -> 17.6; K 3584, N 512, r 32, T 4096 54.1 -> 51.0; three
+// projections of K 3584, T 4096 even. Past that it loses (forward and backward,
+// T 8000: K 1536, N 1536 / 256 / 256 155 -> 165 us), and where the split row
+// projection runs it is not taken. The line is on T, K and r only, so a group
+// computes what its projections would alone.
+constexpr int64_t kFwdOneTokens = 4096;
+bool fwd_one_launch(const Dims& m) { return m.r <= kFwdOpRanks && m.T <= kFwdOneTokens && !fwd_rowsplit(m); }
+
 // bf16 projections whose K or N is not a multiple of 8 (rows not made of
 // 16-byte chunks) run on copies zero-padded to multiples of 8: a padded
 // feature adds exact zeros to every product, so y, dX, dA and dB are the
@@ -491,7 +504,16 @@ hipError_t launch_lora_group_fwd(const mc_lora_desc& d, const void* x, const Lor
         for (int g = 0; g < count; ++g) sumN += Ns[g];
         auto sc = prof::Scope(prof::kLowRank, st, 2.0 * m.T * m.K * m.r * count,
                               2.0 * m.T * m.K + 6.0 * m.T * m.r * count + 12.0 * m.r * (m.K + sumN / count) * count);
-        const bool split = fwd_rowsplit(m);
+        const bool split = fwd_rowsplit(m), one = fwd_one_launch(m);
+        if (one) {
+            FwdOperand ops[kMaxProj];
+            for (int g = 0; g < count; ++g)
+                ops[g] = FwdOperand{proj[g].A, proj[g].B, proj[g].mask, h_save ? h_save[g] : nullptr, Ns[g],
+                                    reinterpret_cast<uint16_t*>(base + w.bt_ext[g])};
+            MC_TRY(launch_lora_fwd_operands(xb, m.T, m.K, m.r, d.scale,
+                                            proj[0].mask ? 1.0f / (1.0f - d.dropout_p) : 1.0f, m.rext, ext_ld, hs, ops,
+                                            count, st));
+        }
         if (split) {
             // One prep launch for every pass (A^T hi / lo, B^T extension
             // operands), one split row projection whose passes share x (run
@@ -533,7 +555,7 @@ hipError_t launch_lora_group_fwd(const mc_lora_desc& d, const void* x, const Lor
             MC_TRY(launch_dy_finish(m.T, m.r, 1.0f, proj[0].mask ? 1.0f / (1.0f - d.dropout_p) : 1.0f, m.rext, ext_ld,
                                     d.scale, fin, count, nullptr, 0, st));
         }
-        for (int p0 = 0, pass = 0; p0 < count && !split; p0 += ppp, ++pass) {
+        for (int p0 = 0, pass = 0; p0 < count && !split && !one; p0 += ppp, ++pass) {
             const int np = count - p0 < ppp ? count - p0 : ppp;
             // A pass holds whole projections; a projection of more than
             // kRowprojMaxRanks ranks (alone in its pass) takes its ranks in

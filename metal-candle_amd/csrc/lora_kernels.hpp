@@ -94,6 +94,22 @@ struct RowprojCall {
 };
 hipError_t launch_rowproj_bf16(const RowprojCall& c, hipStream_t stream);
 
+// The forward's operands of up to kMaxProj projections of one x in one launch:
+// per projection Hd (to h_save [r][T], may be null, and as bf16 scale Hd to
+// columns g rext .. of hs_ext, zeros past r) from A [K][r], and bt_ext [N][rext]
+// from B [r][N] (zeros past r). r <= kFwdOpRanks, K % 8 == 0.
+constexpr int kFwdOpRanks = 32;
+struct FwdOperand {
+    const float* A;
+    const float* B;
+    const uint8_t* mask;  // [T][r] or null
+    float* h_save;
+    int64_t N;
+    uint16_t* bt_ext;
+};
+hipError_t launch_lora_fwd_operands(const uint16_t* x, int64_t T, int64_t K, int r, float scale, float keep, int rext,
+                                    int ext_ld, uint16_t* hs_ext, const FwdOperand* ops, int n, hipStream_t stream);
+
 // The backward's operand pass for up to kMaxProj projections in one launch:
 // per projection the row projection of dY with the fp32 B [r][N] read
 // directly (G = scale dY.B^T, masked, into gd_t [r][T] and the columns of

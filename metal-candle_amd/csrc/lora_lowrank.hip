@@ -1424,6 +1424,116 @@ __global__ __launch_bounds__(64 * kF32RowWaves<RT>) void rowproj_f32(const float
     }
 }
 
+// ------------------------------------------- forward operands in one launch
+// Workgroups [0, tiles * nproj) compute Hd = (x.A) (.) mask / (1-p) of 16
+// tokens of one projection, in fp32 on v_mfma_f32_16x16x4_f32 with A read as
+// stored; the rest write the projections' B^T extension operands. One launch
+// in the place of an operand preparation (A^T split to bf16 hi / lo, B^T) and a
+// row projection that waits for it. Waves take every 16th block of 64 columns;
+// lane l holds columns 8 (l / 16) + q of its token's 32-column groups (16
+// bytes) and the same rows of A for rank l % 16. Every 32 products are summed
+// on their own, these per wave and then the waves as a tree: h is within 1.3e-7
+// of 64 bits (2.5e-6 from the split A). Bound by the latency of one round of
+// loads: at K 1536 a wave has one or two blocks in all, hence 16 waves; 8.2 us
+// cold at T 777 against 5 + 9 for the two launches.
+constexpr int kFwdOpWaves = 16;
+struct FwdOperandsBatch {
+    FwdOperand op[kMaxProj];
+    PrepJob prep[kMaxProj];
+    int64_t start[kMaxProj + 1];  // prep jobs, in 8-element groups
+    const uint16_t* x;
+    int64_t T, K, tiles;
+    int nproj, r, rext, ext_ld;
+    float keep, scale;
+    uint16_t* hs_ext;
+};
+template <int RT>
+__global__ __launch_bounds__(64 * kFwdOpWaves) void lora_fwd_operands(FwdOperandsBatch b) {
+    constexpr int NT = 64 * kFwdOpWaves;
+    const int tid = (int)threadIdx.x;
+    const int64_t blk = blockIdx.x, nh = b.tiles * b.nproj;
+    if (blk >= nh) {  // workgroup-uniform
+        const int64_t n = b.start[b.nproj];
+        for (int64_t idx = (blk - nh) * NT + tid; idx < n; idx += ((int64_t)gridDim.x - nh) * NT) {
+            int j = 0;
+            while (j + 1 < b.nproj && idx >= b.start[j + 1]) ++j;
+            prep_one8(b.prep[j], idx - b.start[j]);
+        }
+        return;
+    }
+    const int pj = (int)(blk / b.tiles);
+    const FwdOperand& P = b.op[pj];
+    const int64_t t0 = (blk % b.tiles) * 16, T = b.T, K = b.K;
+    const int lane = lane_id(), wave = wave_id(), l16 = lane & 15, g = lane >> 4, r = b.r;
+    const uint16_t* xr = b.x + (t0 + l16 < T ? t0 + l16 : T - 1) * K;  // rows past T are dropped below
+    struct Block {
+        uint4 x[2];
+        float a[RT][2][8];
+    };
+    // clamped addresses; columns past K (K % 8 == 0: eight at a time) and ranks
+    // past r are zeroed where they are used
+    auto fetch = [&](int64_t c0, Block& f) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int64_t c = c0 + 32 * i + 8 * g, cc = c < K ? c : K - 8;
+            f.x[i] = *reinterpret_cast<const uint4*>(xr + cc);
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const int j = 16 * rt + l16;
+                const float* pa = P.A + cc * r + (j < r ? j : r - 1);
+#pragma unroll
+                for (int q = 0; q < 8; ++q) f.a[rt][i][q] = pa[(int64_t)q * r];
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // every load goes out before the products
+    };
+    f32x4 tot[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) tot[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    Block cur, next;
+    int64_t c0 = 64 * (int64_t)wave;
+    if (c0 < K) fetch(c0, cur);
+    for (; c0 < K; c0 += 64 * kFwdOpWaves) {
+        if (c0 + 64 * kFwdOpWaves < K) fetch(c0 + 64 * kFwdOpWaves, next);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const bool in = c0 + 32 * i + 8 * g < K;
+            const uint32_t xw[4] = {cur.x[i].x, cur.x[i].y, cur.x[i].z, cur.x[i].w};
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const bool use = in && 16 * rt + l16 < r;
+                f32x4 part = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    const float xv = q & 1 ? bf16_hi(xw[q >> 1]) : bf16_lo(xw[q >> 1]);
+                    part = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? xv : 0.f, use ? cur.a[rt][i][q] : 0.f, part, 0, 0, 0);
+                }
+                tot[rt] += part;
+            }
+        }
+        cur = next;
+    }
+    // accumulator i of lane l is token 4 (l / 16) + i, rank l % 16
+    __shared__ float red[kFwdOpWaves][RT][16][17];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) red[wave][rt][4 * g + i][l16] = tot[rt][i];
+    __syncthreads();
+    for (int o = tid; o < 256 * RT; o += NT) {
+        const int rt = o >> 8, tl = o & 15, jl = (o >> 4) & 15, j = 16 * rt + jl;
+        const int64_t t = t0 + tl;
+        if (t >= T || j >= b.rext) continue;
+        float v = 0.f;
+        if (j < r) {
+            v = wave_tree(kFwdOpWaves, [&](int w) { return red[w][rt][tl][jl]; });
+            if (P.mask) v = P.mask[t * r + j] ? v * b.keep : 0.f;
+            if (P.h_save) P.h_save[(int64_t)j * T + t] = v;
+        }
+        b.hs_ext[t * b.ext_ld + pj * b.rext + j] = f32_to_bf16(b.scale * v);
+    }
+}
+
 // fp32 column reduction out[j][c] = scale * sum_t Pt[j][t] X[t][c] (or out
 // [c][j] with transpose_out) on v_mfma_f32_16x16x4_f32: a workgroup owns 64
 // columns and 16 RT ranks, its waves take every nw-th block of 16 tokens. Lane
@@ -2018,6 +2128,29 @@ hipError_t launch_rowproj_f32(const float* X, int64_t T, int64_t C, const float*
     };
     if (transpose_p) by_rank(std::true_type{});
     else by_rank(std::false_type{});
+    return hipGetLastError();
+}
+
+hipError_t launch_lora_fwd_operands(const uint16_t* x, int64_t T, int64_t K, int r, float scale, float keep, int rext,
+                                    int ext_ld, uint16_t* hs_ext, const FwdOperand* ops, int n, hipStream_t stream) {
+    if (n < 1 || n > kMaxProj || r > kFwdOpRanks) return hipErrorInvalidValue;
+    FwdOperandsBatch b{};
+    b.x = x; b.T = T; b.K = K; b.tiles = (T + 15) / 16;
+    b.nproj = n; b.r = r; b.rext = rext; b.ext_ld = ext_ld;
+    b.keep = keep; b.scale = scale;
+    b.hs_ext = hs_ext;
+    for (int g = 0; g < n; ++g) {
+        b.op[g] = ops[g];
+        PrepJob& j = b.prep[g];
+        j.src = ops[g].B; j.ld_src = ops[g].N; j.valid_rows = ops[g].N; j.valid_cols = r; j.transpose = true;
+        j.hi = ops[g].bt_ext; j.rows_out = ops[g].N; j.cols_out = rext; j.ld_out = rext;
+        if (!prep_vec8(j)) return hipErrorInvalidValue;
+        b.start[g + 1] = b.start[g] + j.rows_out * (rext / 8);
+    }
+    const int64_t nprep = std::min<int64_t>((b.start[n] + 64 * kFwdOpWaves - 1) / (64 * kFwdOpWaves), 256);
+    const dim3 grid((unsigned)(b.tiles * n + nprep));
+    if (r <= 16) lora_fwd_operands<1><<<grid, 64 * kFwdOpWaves, 0, stream>>>(b);
+    else lora_fwd_operands<2><<<grid, 64 * kFwdOpWaves, 0, stream>>>(b);
     return hipGetLastError();
 }
 
