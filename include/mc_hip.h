@@ -228,8 +228,9 @@ mc_status mc_softmax_bwd(int64_t rows, int64_t dim, int64_t causal_rows, int32_t
  * [B, H, S] fp32 (may be NULL) receives the natural log-sum-exp of each score
  * row, which mc_attention_bwd takes.
  * bf16 with D = 64 or 128 runs the MFMA (flash) kernel and needs the
- * workspace of mc_attention_fwd_workspace_size(); other D (<= 256) and fp32
- * run a one-wave-per-row kernel with no workspace. */
+ * workspace of mc_attention_fwd_workspace_size(); fp32 with
+ * D % 4 == 0, D <= 128 runs on the fp32 matrix cores (a backward workspace
+ * only); other D (<= 256) run a one-wave-per-row kernel. */
 typedef struct mc_attn_desc {
     int64_t batch;     /* B >= 1 */
     int64_t seq;       /* S >= 1: queries and keys (self-attention, no KV cache) */

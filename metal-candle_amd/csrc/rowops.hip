@@ -19,8 +19,7 @@
 // the rows whose target is not ignore_index, negated; with smoothing s,
 // (1 - s) * that + s * (-mean of every log-probability of every row).
 // Vocabulary rows are long (10^5 entries), so these use one workgroup (256 or
-// 1024 threads)
-// per row with an online (max, sum) per thread, combined in a
+// 1024 threads) per row with an online (max, sum) per thread, combined in a
 // fixed order. The loss is a second, single-workgroup pass over the per-row
 // values in row order, so it is bitwise reproducible.
 #include <type_traits>
