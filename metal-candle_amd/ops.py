@@ -22,6 +22,10 @@ def _ptr(t):
 
 
 def _stream(t):
+    # The raw handle (0.1 us) and not a Stream object around it (1.9 us of a
+    # 15 us decode call); current_stream refuses what is not on a GPU.
+    if t.is_cuda:
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(t.get_device()))
     return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
 
 
