@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "ring_offsets.hpp"
+
 namespace mc {
 
 constexpr int kWave = 64;
@@ -121,10 +123,9 @@ __device__ __forceinline__ int lane_id() { return threadIdx.x & (kWave - 1); }
 // Raw buffer resource (gfx9 layout, stride 0) over [base, base + bytes):
 // loads at byte offsets >= num_records return zeros (loads into LDS write
 // zeros) and stores there are dropped, which gives branch-free bounds
-// handling. kOOB is an offset that is always out of range. num_records is
+// handling. kOOB (ring_offsets.hpp) is always out of range. num_records is
 // 32-bit: callers keep every offset below 2^31 by basing the resource at
 // the block of rows a workgroup touches.
-constexpr uint32_t kOOB = 0x80000000u;
 // Cache-policy bits of a buffer store (the builtins' aux operand, gfx950
 // encoding): nt, a non-temporal (streaming) store that leaves no dirty line
 // in L2. Used for outputs written as whole 128-byte lines and not read again

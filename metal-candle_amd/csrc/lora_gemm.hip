@@ -763,10 +763,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tiled(int64_t M, int64_t N, F
     uint32_t offk[2];  // NN: k rows 8 wave + 4 j + lane / 16
     if constexpr (NN) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const uint32_t row = (uint32_t)(8 * wave + 4 * j + (lane >> 4));
-            offk[j] = (row * (uint32_t)s0.ldb + 4u * (uint32_t)((lane & 15) ^ (8 * j))) * 4u;
-        }
+        for (int j = 0; j < 2; ++j) offk[j] = nn_chunk_offset(wave, lane, j, (uint32_t)s0.ldb, N - n0);
     } else {
         offb.init(ldb2, tid);
     }
@@ -1232,6 +1229,7 @@ bool gemm_f32_large(int64_t M, int64_t N, bool nn, const GemmSegF32& s0, const G
     constexpr int64_t kLim = ((int64_t)1 << 31) - 256;
     auto rows_fit = [&](int64_t ld, int64_t k) { return (63 * ld + k) * 4 < kLim; };
     if (s0.k < 4 || s0.k % 4 != 0 || s0.lda % 4 != 0 || s0.ldb % 4 != 0) return false;
+    if (nn && N % 4 != 0) return false;
     if ((reinterpret_cast<uintptr_t>(s0.a) | reinterpret_cast<uintptr_t>(s0.b)) & 15) return false;
     if (!rows_fit(s0.lda, s0.k) || !rows_fit(s1.lda, s1.k)) return false;
     if (nn ? (s0.k + 32) * s0.ldb * 4 >= kLim || !rows_fit(s1.ldb, s1.k)

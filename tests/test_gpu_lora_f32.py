@@ -47,6 +47,7 @@ def check_lora(mc, c, scale, p):
     (4100, 64, 1000, 64, 0.0),      # two steps: less than the ring
     (4100, 32, 1000, 7, 0.0),       # one step
     (4100, 1000, 36, 1, 0.0),       # the backward's reduction of one ragged step
+    (4100, 1000, 1024, 8, 0.0),     # ragged columns whose last k row is in a full step
     (4100, 1000, 100, 130, 0.0),    # three blocks of ranks, the last of two
     (1030, 1028, 1028, 65, 0.1),
 ])
