@@ -33,6 +33,7 @@
 
 #include "common.hpp"
 #include "lora_kernels.hpp"
+#include "rules.hpp"
 
 namespace mc {
 namespace {
@@ -1341,7 +1342,7 @@ __device__ __forceinline__ float wave_tree(int nw, F&& v) {
 // of x and four lanes a 64-byte segment; the next block is requested before a
 // block is multiplied. Bound by the reads of x: the one workgroup per token
 // that it replaces read all of P for each token (2036 x 8960, r 16: 280 -> 51
-// us; 2036 x 1536: 106 -> 12 us; 512 x 768, r 8: 10 -> 6.5 us).
+// us; 2036 x 1536: 106 -> 12 us; 512 x 768, r 8: 10 -> 6 us).
 // Every 16 products are summed on their own, the 16s in pairs, these per wave
 // and then the waves in order.
 template <int RT> constexpr int kF32RowWaves = RT <= 2 ? 16 : 8;  // 128 or 256 registers per lane
@@ -1361,25 +1362,42 @@ __global__ __launch_bounds__(64 * kF32RowWaves<RT>) void rowproj_f32(const float
     struct Block {
         f32x4 x[2 * NB], p[RT][2 * NB];
     };
+    // Ranks past r read rank r - 1's and are zeroed where they are used: a select
+    // here would wait for the loads.
     auto fetch = [&](int64_t c0, Block& f) {
-        const bool whole = c0 + W <= C;  // wave-uniform
+        if (c0 + W <= C) {  // wave-uniform
+#pragma unroll
+            for (int i = 0; i < 2 * NB; ++i) {
+                const int64_t c = c0 + 16 * i;
+                f.x[i] = load4(xr + c);
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {
+                    const int j = j0 + 16 * rt + l16, jc = j < r ? j : r - 1;
+                    if constexpr (TP) {
+                        const float* pr = P + (c + 4 * g) * r + jc;
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) f.p[rt][i][q] = pr[(int64_t)q * r];
+                    } else {
+                        f.p[rt][i] = load4(P + (int64_t)jc * C + c + 4 * g);
+                    }
+                }
+            }
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < 2 * NB; ++i) {
             const int64_t c = c0 + 16 * i, left = C - c - 4 * g;
-            f.x[i] = whole ? load4(xr + c) : load4_n(xr + c, left);
+            f.x[i] = load4_n(xr + c, left);
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) {
                 const int j = j0 + 16 * rt + l16, jc = j < r ? j : r - 1;
                 if constexpr (TP) {
                     const float* pr = P + (c + 4 * g) * r + jc;
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) f.p[rt][i][q] = whole || q < left ? pr[(int64_t)q * r] : 0.f;
+                    for (int q = 0; q < 4; ++q) f.p[rt][i][q] = q < left ? pr[(int64_t)q * r] : 0.f;
                 } else {
-                    const float* pr = P + (int64_t)jc * C + c + 4 * g;
-                    f.p[rt][i] = whole ? load4(pr) : load4_n(pr, left);
+                    f.p[rt][i] = load4_n(P + (int64_t)jc * C + c + 4 * g, left);
                 }
-#pragma unroll
-                for (int q = 0; q < 4; ++q) f.p[rt][i][q] = j < r ? f.p[rt][i][q] : 0.f;
             }
         }
     };
@@ -1399,7 +1417,8 @@ __global__ __launch_bounds__(64 * kF32RowWaves<RT>) void rowproj_f32(const float
                 part[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
-                    part[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.x[i][q], cur.p[rt][i][q], part[i], 0, 0, 0);
+                    part[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                        cur.x[i][q], j0 + 16 * rt + l16 < r ? cur.p[rt][i][q] : 0.f, part[i], 0, 0, 0);
             }
             if constexpr (NB == 2) tot[rt] += (part[0] + part[1]) + (part[2] + part[3]);
             else tot[rt] += part[0] + part[1];
@@ -1418,6 +1437,45 @@ __global__ __launch_bounds__(64 * kF32RowWaves<RT>) void rowproj_f32(const float
         const int64_t t = t0 + tl;
         if (t >= T || j >= r) continue;
         float v = scale * wave_tree(nw, [&](int w) { return red[w][rt][tl][jl]; });
+        if (mask) v = mask[t * r + j] ? v * keep : 0.f;
+        if (out_t) out_t[(int64_t)j * T + t] = v;
+        if (out_ext) out_ext[t * r + j] = v * ext_scale;
+    }
+}
+
+// The row projection of few tokens and at most 4 ranks (rowproj_f32_by_token): a
+// workgroup per token, thread i taking columns i, i + 256, ... in order; then
+// the lanes, then the waves in order. K 8960, r 4, T 32, with the product after
+// it: 14.8 us, 28.6 on the 16-token tiles.
+template <bool TP>
+__global__ __launch_bounds__(256) void rowproj_f32_rows(const float* __restrict__ X, int64_t T, int64_t C,
+                                                        const float* __restrict__ P, int r, float scale,
+                                                        const uint8_t* __restrict__ mask, float keep,
+                                                        float* __restrict__ out_t, float* __restrict__ out_ext,
+                                                        float ext_scale) {
+    constexpr int R = 4;
+    const int64_t t = blockIdx.x;
+    const float* xr = X + t * C;
+    float acc[R] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int64_t c = threadIdx.x; c < C; c += 256) {
+        const float xv = xr[c];
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            const int jc = j < r ? j : r - 1;  // ranks past r are dropped below
+            acc[j] += xv * (TP ? P[c * r + jc] : P[(int64_t)jc * C + c]);
+        }
+    }
+    __shared__ float red[4][R];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const float v = wave_sum(acc[j]);
+        if (lane_id() == 0) red[wave_id()][j] = v;
+    }
+    __syncthreads();
+    const int j = (int)threadIdx.x;
+    if (j < r) {
+        float v = scale * ((red[0][j] + red[1][j]) + (red[2][j] + red[3][j]));
         if (mask) v = mask[t * r + j] ? v * keep : 0.f;
         if (out_t) out_t[(int64_t)j * T + t] = v;
         if (out_ext) out_ext[t * r + j] = v * ext_scale;
@@ -2112,6 +2170,14 @@ hipError_t launch_rowproj_f32(const float* X, int64_t T, int64_t C, const float*
                               int r, float scale, const uint8_t* mask, float keep, float* out_t,
                               float* out_ext, float ext_scale, hipStream_t stream) {
     if (T >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
+    if (rowproj_f32_by_token(T, r)) {
+        const dim3 grid((unsigned)T);
+        if (transpose_p)
+            rowproj_f32_rows<true><<<grid, 256, 0, stream>>>(X, T, C, P, r, scale, mask, keep, out_t, out_ext, ext_scale);
+        else
+            rowproj_f32_rows<false><<<grid, 256, 0, stream>>>(X, T, C, P, r, scale, mask, keep, out_t, out_ext, ext_scale);
+        return hipGetLastError();
+    }
     auto go = [&](auto rt_tag, auto tp_tag) {
         constexpr int RT = decltype(rt_tag)::value;
         constexpr bool TP = decltype(tp_tag)::value;

@@ -71,6 +71,14 @@ def test_lora_f32_rank_products(mc, dev, T, K, N, r):
     check_lora(mc, lora_case(dev, T, K, N, r, 0.1, T + K + r), 2.0, 0.1)
 
 
+@pytest.mark.parametrize("T,K,N,r", [(2048, 300, 7, 1), (2049, 300, 7, 1), (33, 1030, 513, 3), (512, 255, 257, 4),
+                                     (513, 256, 255, 4), (256, 8960, 512, 2)])
+def test_lora_f32_projection_by_token(mc, dev, T, K, N, r):
+    """The row projection with a workgroup per token, and just past it: up to 4
+    ranks and 2048 tokens over the ranks, columns around a pass of 256."""
+    check_lora(mc, lora_case(dev, T, K, N, r, 0.1, T + K + r), 2.0, 0.1)
+
+
 def test_lora_f32_ring_gemm_sees_only_its_rows(mc, dev):
     """A non-finite token reaches its own row of y and dX and no other, and a
     non-finite weight row its own column of y."""
