@@ -1593,16 +1593,18 @@ __global__ __launch_bounds__(64 * kFwdOpWaves) void lora_fwd_operands(FwdOperand
 }
 
 // fp32 column reduction out[j][c] = scale * sum_t Pt[j][t] X[t][c] (or out
-// [c][j] with transpose_out) on v_mfma_f32_16x16x4_f32: a workgroup owns 64
+// [c][j] with transpose_out) on v_mfma_f32_16x16x4_f32: a workgroup owns 16 CT
 // columns and 16 RT ranks, its waves take every nw-th block of 16 tokens. Lane
-// l loads columns 4 (l % 16) .. + 3 of token 4 (l / 16) + q (whole 256-byte row
-// segments per 16 lanes), which are the operands of four 16-column tiles, tile
-// e holding columns 4 i + e, and 16 bytes of rank l % 16's row of Pt for the
-// four q. Bound by the reads of X, each rank group one pass over it: 2036
-// tokens, 1536 and 8960 columns, r 16: 53 -> 19 us against 8 ranks x 16
-// columns per workgroup on the vector unit. Every block's products are summed on
-// their own (in two chains of 8 where the registers allow it), the blocks per
-// wave and then the waves in order.
+// l loads columns CT (l % 16) .. of token 4 (l / 16) + q (16 lanes read a row
+// segment of 64 CT bytes), which are the operands of CT 16-column tiles, tile e
+// holding columns CT i + e, and 16 bytes of rank l % 16's row of Pt for the
+// four q. Bound by the reads of X, each rank group one pass over it, and where
+// the output is small by the latency of a workgroup's walk over T; the tile is
+// colreduce_f32_tile's. 2036 tokens, 1536 and 8960 columns, r 16: 53 -> 19 us
+// against 8 ranks x 16 columns per workgroup on the vector unit; 512 tokens, 768
+// columns, r 64: 7.8 us there, 18.3 with 64 x 64 tiles, 4.9 with 16 x 16. Every
+// block's products are summed on their own (in two chains of 8 where RT is 1),
+// the blocks per wave and then the waves in order.
 // One or two reductions (dA over x and dB over dY) in one launch: blocks
 // [0, nblk0) take job 0, the rest job 1.
 struct ColF32Job {
@@ -1615,30 +1617,38 @@ struct ColF32Job {
     int64_t ctiles;
 };
 template <int RT> constexpr int kF32ColWaves = RT == 1 ? 16 : 8;  // 128 or 256 registers per lane
-template <int RT>
+template <int RT, int CT>
 __global__ __launch_bounds__(64 * kF32ColWaves<RT>) void colreduce_f32(int64_t T, int r, ColF32Job ja, ColF32Job jb,
                                                                     int64_t nblk0) {
+    constexpr int COLS = 16 * CT;
     const bool second = (int64_t)blockIdx.x >= nblk0;  // workgroup-uniform
     const ColF32Job& J = second ? jb : ja;
     const int64_t b = (int64_t)blockIdx.x - (second ? nblk0 : 0);
     const float* __restrict__ X = J.X;
     const float* __restrict__ Pt = J.Pt;
     const int64_t C = J.C, ctiles = J.ctiles;
-    const int64_t c0 = (b % ctiles) * 64;
+    const int64_t c0 = (b % ctiles) * COLS;
     const int j0 = (int)(b / ctiles) * 16 * RT;
     const int lane = lane_id(), wave = wave_id(), l16 = lane & 15, g = lane >> 4;
     const int nw = (int)(blockDim.x >> 6);
-    const int64_t cleft = C - c0 - 4 * l16;
+    const int64_t cleft = C - c0 - CT * l16;
+    typedef float vec __attribute__((ext_vector_type(CT)));
     struct Block {
-        f32x4 x[4], a[RT];
+        vec x[4];
+        f32x4 a[RT];
     };
     auto fetch = [&](int64_t t0, Block& f) {
         const int64_t tleft = T - t0 - 4 * g;
-        const bool whole = t0 + 16 <= T && c0 + 64 <= C;  // wave-uniform
-        const float* xr = X + (t0 + 4 * g) * C + c0 + 4 * l16;
+        const bool whole = t0 + 16 <= T && (CT == 1 || c0 + COLS <= C);  // wave-uniform
+        // CT == 1: columns past C read the last one's and are dropped below
+        const float* xr = X + (t0 + 4 * g) * C + (CT == 1 && cleft < 1 ? C - 1 : c0 + CT * l16);
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            f.x[q] = whole ? load4(xr + (int64_t)q * C) : load4_n(xr + (int64_t)q * C, q < tleft ? cleft : 0);
+        for (int q = 0; q < 4; ++q) {
+            if constexpr (CT == 4)
+                f.x[q] = whole ? load4(xr + (int64_t)q * C) : load4_n(xr + (int64_t)q * C, q < tleft ? cleft : 0);
+            else
+                f.x[q][0] = whole || q < tleft ? xr[(int64_t)q * C] : 0.f;
+        }
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
             const int j = j0 + 16 * rt + l16;
@@ -1647,11 +1657,11 @@ __global__ __launch_bounds__(64 * kF32ColWaves<RT>) void colreduce_f32(int64_t T
         }
     };
     constexpr int NC = RT == 1 ? 2 : 1;  // chains
-    f32x4 tot[RT][4];
+    f32x4 tot[RT][CT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) tot[rt][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int e = 0; e < CT; ++e) tot[rt][e] = f32x4{0.f, 0.f, 0.f, 0.f};
     Block cur, next;
     int64_t t0 = 16 * (int64_t)wave;
     if (t0 < T) fetch(t0, cur);
@@ -1659,34 +1669,39 @@ __global__ __launch_bounds__(64 * kF32ColWaves<RT>) void colreduce_f32(int64_t T
         if (t0 + 16 * nw < T) fetch(t0 + 16 * nw, next);
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-            f32x4 part[NC][4];
+            f32x4 part[NC][CT];
 #pragma unroll
             for (int q = 0; q < 4; ++q)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
+                for (int e = 0; e < CT; ++e) {
                     f32x4& p = part[q * NC / 4][e];
                     const f32x4 c = q % (4 / NC) == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : p;
                     p = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.a[rt][q], cur.x[q][e], c, 0, 0, 0);
                 }
 #pragma unroll
-            for (int e = 0; e < 4; ++e) tot[rt][e] += NC == 2 ? part[0][e] + part[NC - 1][e] : part[0][e];
+            for (int e = 0; e < CT; ++e) tot[rt][e] += NC == 2 ? part[0][e] + part[NC - 1][e] : part[0][e];
         }
         cur = next;
     }
-    // accumulator i of tile e is rank 4 (l / 16) + i, column 4 (l % 16) + e;
-    // LDS rows of 68 floats keep both the 16-byte writes and the transposed
-    // reads off each other's banks
-    __shared__ __attribute__((aligned(16))) float red[kF32ColWaves<RT>][16][68];
+    // accumulator i of tile e is rank 4 (l / 16) + i, column CT (l % 16) + e;
+    // LDS rows of 68 (17) floats keep both the writes and the transposed reads
+    // off each other's banks
+    __shared__ __attribute__((aligned(16))) float red[kF32ColWaves<RT>][16][CT == 4 ? 68 : 17];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
         if (rt > 0) __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            *reinterpret_cast<f32x4*>(&red[wave][4 * g + i][4 * l16]) =
-                f32x4{tot[rt][0][i], tot[rt][1][i], tot[rt][2][i], tot[rt][3][i]};
+        for (int i = 0; i < 4; ++i) {
+            if constexpr (CT == 4)
+                *reinterpret_cast<f32x4*>(&red[wave][4 * g + i][4 * l16]) =
+                    f32x4{tot[rt][0][i], tot[rt][1][i], tot[rt][2][i], tot[rt][3][i]};
+            else
+                red[wave][4 * g + i][l16] = tot[rt][0][i];
+        }
         __syncthreads();
-        for (int o = (int)threadIdx.x; o < 1024; o += (int)blockDim.x) {
-            const int jl = J.transpose_out ? o & 15 : o >> 6, cl = J.transpose_out ? o >> 4 : o & 63;
+        for (int o = (int)threadIdx.x; o < 16 * COLS; o += (int)blockDim.x) {
+            constexpr int LC = CT == 4 ? 6 : 4;  // log2 of the columns
+            const int jl = J.transpose_out ? o & 15 : o >> LC, cl = J.transpose_out ? o >> 4 : o & (COLS - 1);
             const int j = j0 + 16 * rt + jl;
             const int64_t c = c0 + cl;
             if (j >= r || c >= C) continue;
@@ -2222,26 +2237,31 @@ hipError_t launch_lora_fwd_operands(const uint16_t* x, int64_t T, int64_t K, int
 
 hipError_t launch_colreduce_f32(const ColF32Call* calls, int n, int64_t T, int r, hipStream_t stream) {
     if (n < 1 || n > 2) return hipErrorInvalidValue;
-    const int rt = r <= 16 ? 1 : r <= 32 ? 2 : 4;
+    int64_t cols = 0;
+    for (int i = 0; i < n; ++i) cols += calls[i].C;
+    const ColF32Tile tile = colreduce_f32_tile(T, cols, r);
+    const int width = 16 * tile.ct, ranks = 16 * tile.rt;
     ColF32Job j[2]{};
     int64_t nblk[2] = {0, 0};
     for (int i = 0; i < n; ++i) {
         const ColF32Call& c = calls[i];
-        j[i] = ColF32Job{c.X, c.C, c.Pt, c.scale, c.transpose_out ? 1 : 0, c.out, (c.C + 63) / 64};
-        nblk[i] = j[i].ctiles * ((r + 16 * rt - 1) / (16 * rt));
+        j[i] = ColF32Job{c.X, c.C, c.Pt, c.scale, c.transpose_out ? 1 : 0, c.out, (c.C + width - 1) / width};
+        nblk[i] = j[i].ctiles * ((r + ranks - 1) / ranks);
     }
     if (nblk[0] + nblk[1] >= ((int64_t)1 << 31)) return hipErrorInvalidValue;
     if (nblk[0] + nblk[1] == 0) return hipSuccess;
     const dim3 grid((unsigned)(nblk[0] + nblk[1]));
     const ColF32Job& jb = n > 1 ? j[1] : j[0];
-    auto go = [&](auto rt_tag) {
-        constexpr int RT = decltype(rt_tag)::value;
+    auto go = [&](auto rt_tag, auto ct_tag) {
+        constexpr int RT = decltype(rt_tag)::value, CT = decltype(ct_tag)::value;
         const int nw = (int)std::min<int64_t>(kF32ColWaves<RT>, (T + 15) / 16);  // a wave per 16 tokens
-        colreduce_f32<RT><<<grid, 64 * nw, 0, stream>>>(T, r, j[0], jb, nblk[0]);
+        colreduce_f32<RT, CT><<<grid, 64 * nw, 0, stream>>>(T, r, j[0], jb, nblk[0]);
     };
-    if (rt == 1) go(std::integral_constant<int, 1>{});
-    else if (rt == 2) go(std::integral_constant<int, 2>{});
-    else go(std::integral_constant<int, 4>{});
+    constexpr std::integral_constant<int, 4> wide{};
+    if (tile.ct == 1) go(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
+    else if (tile.rt == 1) go(std::integral_constant<int, 1>{}, wide);
+    else if (tile.rt == 2) go(std::integral_constant<int, 2>{}, wide);
+    else go(std::integral_constant<int, 4>{}, wide);
     return hipGetLastError();
 }
 

@@ -15,6 +15,10 @@ SOURCE = """
 #include "rules.hpp"
 extern "C" {
 int rowproj_f32_by_token(int64_t T, int r) { return mc::rowproj_f32_by_token(T, r); }
+int colreduce_f32_tile(int64_t T, int64_t cols, int r) {
+    const mc::ColF32Tile t = mc::colreduce_f32_tile(T, cols, r);
+    return 10 * t.rt + t.ct;
+}
 }
 """
 
@@ -41,3 +45,22 @@ def rules(tmp_path_factory):
 def test_rowproj_f32_by_token(rules, r, K, T, by_token, by_16):
     chosen = by_token if rules.rowproj_f32_by_token(ctypes.c_int64(T), r) else by_16
     assert chosen <= 1.03 * min(by_token, by_16)
+
+
+# dB of one projection, us, by tile (10 rt + ct).
+@pytest.mark.parametrize("r,cols,T,us", [
+    (4, 128, 2048, {11: 8.1, 14: 15.6}), (4, 4608, 2048, {11: 22.9, 14: 18.5}), (4, 8960, 512, {11: 10.7, 14: 7.8}),
+    (16, 128, 4096, {11: 15.9, 14: 28.0}), (16, 768, 32, {11: 2.9, 14: 4.5}), (16, 2304, 2048, {11: 10.9, 14: 16.9}),
+    (16, 4608, 32, {11: 3.2, 14: 4.5}), (16, 4608, 2048, {11: 25.8, 14: 20.6}), (16, 8960, 4096, {11: 74.1, 14: 43.2}),
+    (32, 128, 512, {11: 4.4, 14: 6.3, 21: 5.7, 24: 10.2}), (32, 2304, 2048, {11: 15.5, 14: 17.0, 21: 17.2, 24: 31.3}),
+    (32, 4608, 2048, {11: 29.7, 14: 20.0, 21: 33.7, 24: 35.7}), (32, 8960, 4096, {11: 104.9, 14: 72.4, 21: 96.5, 24: 67.7}),
+    (64, 128, 512, {11: 4.5, 14: 6.3, 24: 10.3, 44: 17.6}), (64, 768, 4096, {11: 16.6, 14: 29.1, 24: 56.0, 44: 92.0}),
+    (64, 1536, 32, {11: 3.2, 14: 4.6, 24: 6.5, 44: 10.6}), (64, 1536, 2048, {11: 15.7, 14: 17.4, 24: 31.3, 44: 50.9}),
+    (64, 2304, 2048, {11: 22.9, 14: 17.8, 24: 31.7, 44: 51.2}), (64, 4608, 2048, {11: 50.2, 14: 33.0, 24: 35.9, 44: 56.2}),
+    (64, 8960, 2048, {11: 94.1, 14: 59.1, 24: 57.5, 44: 57.6}), (64, 8960, 4096, {11: 187.9, 14: 110.4, 24: 107.4, 44: 103.1}),
+    (128, 768, 4096, {11: 26.0, 14: 29.1, 24: 56.5, 44: 91.8}), (128, 4608, 4096, {11: 189.1, 14: 85.8, 24: 102.2, 44: 99.7}),
+    (128, 8960, 2048, {11: 180.2, 14: 98.1, 24: 82.5, 44: 104.4}),
+])
+def test_colreduce_f32_tile(rules, r, cols, T, us):
+    tile = rules.colreduce_f32_tile(ctypes.c_int64(T), ctypes.c_int64(cols), r)
+    assert us[tile] <= 1.03 * min(us.values())

@@ -71,6 +71,14 @@ def test_lora_f32_rank_products(mc, dev, T, K, N, r):
     check_lora(mc, lora_case(dev, T, K, N, r, 0.1, T + K + r), 2.0, 0.1)
 
 
+@pytest.mark.parametrize("T,K,N,r", [(65, 3070, 67, 16), (300, 3001, 130, 7), (32, 6300, 65, 40), (33, 6300, 65, 40),
+                                     (270, 6211, 90, 33), (4099, 6211, 90, 64), (4096, 6200, 64, 65)])
+def test_lora_f32_column_tiles(mc, dev, T, K, N, r):
+    """The column reductions' other tiles (64 columns by 16, 32 and 64 ranks):
+    wide inputs of ragged columns, tokens and ranks."""
+    check_lora(mc, lora_case(dev, T, K, N, r, 0.1, T + K + r), 2.0, 0.1)
+
+
 @pytest.mark.parametrize("T,K,N,r", [(2048, 300, 7, 1), (2049, 300, 7, 1), (33, 1030, 513, 3), (512, 255, 257, 4),
                                      (513, 256, 255, 4), (256, 8960, 512, 2)])
 def test_lora_f32_projection_by_token(mc, dev, T, K, N, r):
