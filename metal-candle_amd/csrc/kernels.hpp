@@ -99,7 +99,6 @@ hipError_t launch_lora_group_bwd(const mc_lora_desc& d, const void* x, const Lor
 
 // The grouped forward of a few tokens (lora_small.hip), with its own partial
 // sums in ws (lora_small_ws bytes).
-constexpr int kSmallTokens = 32, kSmallRanks = 64;
 size_t lora_small_ws(int64_t T, int64_t K, int r, int count);
 hipError_t launch_lora_small_fwd(const mc_lora_desc& d, const void* x, const LoraProj* proj, int count, void* const* y,
                                  float* const* h_save, void* ws, hipStream_t stream);

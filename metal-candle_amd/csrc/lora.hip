@@ -19,6 +19,7 @@
 #include "kernels.hpp"
 #include "lora_kernels.hpp"
 #include "profile.hpp"
+#include "rules.hpp"
 
 namespace mc {
 namespace {
@@ -122,10 +123,20 @@ bool bwd_rowsplit(const Dims& m, const int64_t* N, int count) {
 // operand path, whose per-step operand split is the kernel's bottleneck.
 bool bwd_colsplit(const Dims& m, const int64_t* N, int count) { return bwd_rowsplit(m, N, count) && m.T % 8 == 0; }
 
-// Few tokens take two launches that read W row by row instead of the tiled
-// path's three. A rule on the tokens and ranks only, so a grouped call still
-// computes the sums of single calls.
-bool fwd_small(const Dims& m) { return m.bf16 && m.T <= kSmallTokens && m.r <= kSmallRanks; }
+// Few tokens take launches that read W row by row instead of the tiled path's.
+bool fwd_small(const Dims& m, int64_t N) { return m.bf16 && lora_few_tokens(m.T, N, m.r); }
+
+// A group's projections by the path that each takes: sel holds the few-token
+// ones, then the others, each in the group's order; returns the first kind's count.
+int few_first(const Dims& m, const int64_t* N, int count, int (&sel)[kMaxProj]) {
+    int n = 0, few = 0;
+    for (int g = 0; g < count; ++g)
+        if (fwd_small(m, N[g])) sel[n++] = g;
+    few = n;
+    for (int g = 0; g < count; ++g)
+        if (!fwd_small(m, N[g])) sel[n++] = g;
+    return few;
+}
 
 // The forward's preparation and row projection as one launch
 // (launch_lora_fwd_operands). It reads x once per projection and repeats A's
@@ -313,6 +324,14 @@ LoraGroupFwdWs lora_group_fwd_ws(const mc_lora_desc& d, const int64_t* N, int co
     const Dims m = dims_of(d);
     LoraGroupFwdWs w{};
     size_t off = 0;
+    int sel[kMaxProj];
+    const int few = few_first(m, N, count, sel);
+    if (few > 0 && few < count) {  // the two kinds' calls share the workspace
+        int64_t Ns[kMaxProj];
+        for (int g = 0; g < count; ++g) Ns[g] = N[sel[g]];
+        w.total = std::max(lora_group_fwd_ws(d, Ns, few).total, lora_group_fwd_ws(d, Ns + few, count - few).total);
+        return w;
+    }
     const int ppp = proj_per_pass(m.r);
     for (int p0 = 0, pass = 0; p0 < count; p0 += ppp, ++pass) {
         const int np = count - p0 < ppp ? count - p0 : ppp;
@@ -331,7 +350,7 @@ LoraGroupFwdWs lora_group_fwd_ws(const mc_lora_desc& d, const int64_t* N, int co
         off += align256((size_t)npass * rowsplit_splits(m.T, m.K) * m.T * ld * 4);
     }
     w.small = off;
-    if (fwd_small(m)) off += align256(lora_small_ws(m.T, m.K, m.r, count));
+    if (few > 0) off += align256(lora_small_ws(m.T, m.K, m.r, count));
     w.total = off;
     return w;
 }
@@ -487,10 +506,26 @@ hipError_t launch_lora_group_fwd(const mc_lora_desc& d, const void* x, const Lor
     const Dims m = dims_of(d);
     int64_t Ns[kMaxProj];
     for (int g = 0; g < count; ++g) Ns[g] = proj[g].N;
+    int sel[kMaxProj];
+    const int few = few_first(m, Ns, count, sel);
+    if (few > 0 && few < count) {  // both kinds: a call each, the second in the first's workspace
+        for (int first = 0, n = few; first < count; first += n, n = count - few) {
+            LoraProj p[kMaxProj];
+            void* yy[kMaxProj];
+            float* hh[kMaxProj];
+            for (int i = 0; i < n; ++i) {
+                p[i] = proj[sel[first + i]];
+                yy[i] = y[sel[first + i]];
+                hh[i] = h_save ? h_save[sel[first + i]] : nullptr;
+            }
+            MC_TRY(launch_lora_group_fwd(d, x, p, n, yy, hh, ws, st));
+        }
+        return hipSuccess;
+    }
     const LoraGroupFwdWs w = lora_group_fwd_ws(d, Ns, count);
     char* base = static_cast<char*>(ws);
     const uint16_t* xb = static_cast<const uint16_t*>(x);
-    if (fwd_small(m)) {
+    if (few > 0) {
         int64_t sumN = 0;
         for (int g = 0; g < count; ++g) sumN += Ns[g];
         auto sc = gemm_scope(st, m.T, sumN, m.K, m.r, m.r, 2);

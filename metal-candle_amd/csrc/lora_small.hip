@@ -13,23 +13,23 @@
 //                 term is added in fp32 from the partial sums of H.
 //
 // Bound by the read of W and, for small ones, by launches: the tiled path runs
-// an operand preparation, a row projection and a GEMM whose N / 128 workgroups
-// each walk all of K. Per call in a loop, K -> N, tiled path / this:
-//   T  1,  1536 -> 1536,  r 16   26.6 /  8.6 us
-//   T  1,  3584 -> 18944, r 64   57.3 / 42.8 us (W alone: 22 us at 6.2 TB/s)
-//   T  1, 18944 -> 3584,  r 64    193 / 37.8 us
-//   T 16,  3584 -> 3584,  r 16   50.8 / 14.4 us
-//   T 32,  3584 -> 18944, r 16   56.1 / 53.7 us
-//   T 32, 18944 -> 3584,  r 64    200 / 89.4 us
-// With four token tiles (T 64) it was ahead on narrow outputs (8960 -> 1536,
-// r 64: 100 / 69 us) and behind on wide ones (3584 -> 18944: 61 / 90 us), and
-// the choice may not depend on N (fwd_small), so the limit is 32.
+// an operand preparation, a row projection (one launch up to 32 ranks and 4095
+// columns) and a GEMM, whose few workgroups each walk all of K. The device's
+// time, inputs not in the caches, tiled path / this, K -> N (the rule between
+// the two is lora_few_tokens):
+//   T  8,  1536 -> 1536,  r 8    16.6 /  9.4 us
+//   T  8,  3584 -> 18944, r 64   56.4 / 50.1 us (W alone: 22 us at 6.2 TB/s)
+//   T  8, 18944 -> 3584,  r 64    134 / 51.8 us
+//   T 16,  3584 -> 3584,  r 8    31.6 / 14.1 us
+//   T 32,  3584 -> 3584,  r 64   39.9 / 30.7 us
+//   T 32, 18944 -> 3584,  r 64    136 / 91.8 us
 #include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
 #include "lora_kernels.hpp"
+#include "rules.hpp"
 
 namespace mc {
 namespace {

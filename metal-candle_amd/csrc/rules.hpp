@@ -7,6 +7,24 @@
 
 namespace mc {
 
+// Few-token LoRA forward (lora_small.hip) for one projection, else the tiled
+// path. A projection of a group takes the path that it would take alone, so
+// that the group's results are those of single calls. Up to 16 tokens it was
+// never the slower of the two by more than 10%; past that its workgroups are 32
+// rows of W, and it is ahead while a round of the CUs holds them all (N 8192).
+// Forward, us, few-token / tiled (before the tiles for small grids):
+//   T 16: 1536 -> 8960, r 8 18.7 / 17.0 (27.6), 3584 -> 18944, r 64 54.2 / 57.4 (66.5)
+//   T 17: 1536 -> 1536, r 8 12.6 / 16.9 (27.8), 3584 -> 18944, r 64 65.3 / 57.3 (66.3)
+//   T 32: 896 -> 896, r 8 10.1 / 11.6 (19.1), 1536 -> 8960, r 8 21.6 / 17.3 (28.1),
+//         18944 -> 3584, r 64 91.8 / 136 (202), 1536 -> 18944, r 64 48.2 / 40.2 (41.6),
+//         3584 -> 3584, r 64 30.7 / 39.9 (51.7), 3584 -> 18944, r 64 71.7 / 60.7 (67.1)
+// Groups, T 32: 1536 -> 8960, 8960, r 64 48.0 / 39.7 (41.0); 3584 -> 18944, 18944
+// gains nothing from the line: r 64 102.6 / 103.5 (104.6), r 16 81.6 / 87.4 (106).
+constexpr int kSmallTokens = 32, kSmallRanks = 64;
+constexpr bool lora_few_tokens(int64_t T, int64_t N, int r) {
+    return r <= kSmallRanks && (T <= 16 || (T <= kSmallTokens && N <= 8192));
+}
+
 // Float32 row projection of few tokens and ranks: a workgroup per token
 // (rowproj_f32_rows) instead of one per 16 tokens, which leaves most CUs
 // without a row to read. Projection and its product, us, per token / per 16:

@@ -14,6 +14,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SOURCE = """
 #include "rules.hpp"
 extern "C" {
+int lora_few_tokens(int64_t T, int64_t N, int r) { return mc::lora_few_tokens(T, N, r); }
 int rowproj_f32_by_token(int64_t T, int r) { return mc::rowproj_f32_by_token(T, r); }
 int colreduce_f32_tile(int64_t T, int64_t cols, int r) {
     const mc::ColF32Tile t = mc::colreduce_f32_tile(T, cols, r);
@@ -32,6 +33,28 @@ def rules(tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", "-I", inc, str(src), "-o", str(so)],
                    check=True)
     return ctypes.CDLL(str(so))
+
+
+# A projection's forward, us: few-token kernels, tiled path, the tiled path before it had tiles for small
+# grids. Up to 16 tokens the rule may leave 10% to the tiled path.
+@pytest.mark.parametrize("T,K,N,r,few,tiled,former", [
+    (8, 1536, 1536, 8, 9.4, 16.6, 27.3), (8, 3584, 18944, 64, 50.1, 56.4, 65.9), (16, 1536, 8960, 8, 18.7, 17.0, 27.6),
+    (16, 18944, 3584, 64, 59.2, 135.0, 198.4), (17, 896, 896, 8, 9.4, 11.5, 19.2), (17, 1536, 8960, 8, 19.3, 17.1, 28.0),
+    (17, 3584, 18944, 64, 65.3, 57.3, 66.3), (20, 8960, 1536, 64, 47.1, 71.0, 98.9), (24, 1536, 8960, 64, 31.7, 29.0, 34.9),
+    (24, 3584, 18944, 8, 51.5, 47.6, 66.5), (24, 3584, 3584, 64, 29.5, 39.8, 51.5), (28, 3584, 512, 8, 20.6, 31.6, 50.6),
+    (32, 896, 128, 64, 19.4, 23.9, 27.6), (32, 1536, 1536, 64, 23.3, 28.0, 33.4), (32, 1536, 18944, 64, 48.2, 40.2, 41.6),
+    (32, 896, 28672, 48, 39.4, 33.4, 33.8), (32, 3584, 18944, 64, 71.7, 60.7, 67.1), (32, 18944, 3584, 8, 77.9, 125.4, 190.4),
+])
+def test_lora_few_tokens(rules, T, K, N, r, few, tiled, former):
+    chosen = few if rules.lora_few_tokens(ctypes.c_int64(T), ctypes.c_int64(N), r) else tiled
+    assert chosen <= (1.1 if T <= 16 else 1.03) * min(few, tiled)
+    assert chosen <= former
+
+
+def test_lora_few_tokens_limits(rules):
+    for T, N, r, want in ((16, 1 << 20, 64, 1), (16, 8, 65, 0), (17, 8192, 64, 1), (17, 8200, 1, 0), (32, 8192, 64, 1),
+                          (33, 8, 1, 0)):
+        assert rules.lora_few_tokens(ctypes.c_int64(T), ctypes.c_int64(N), r) == want
 
 
 # A forward without W (projection and a product of 64 columns), us: workgroup per token, per 16 tokens.

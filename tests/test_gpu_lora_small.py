@@ -64,6 +64,25 @@ def test_lora_few_tokens_group_equals_single(mc, dev, T):
         assert torch.equal(y, y1) and torch.equal(h, h1)
 
 
+@pytest.mark.parametrize("T", [1, 16, 17, 32])
+@pytest.mark.parametrize("Ns,r", [((8960, 8952, 24), 16), ((8184, 8192, 24), 64), ((24, 8200, 1000, 8960), 33)])
+def test_lora_few_tokens_wide_group_equals_single(mc, dev, T, Ns, r):
+    """Groups of 16384 or more columns take the wide kernels where each of their
+    projections alone takes the narrow ones, and past 16 tokens projections of
+    more than 8192 columns go another way than the rest of the group."""
+    K = 264
+    cs = [small_case(dev, T, K, N, r, 0.1, i % 2 == 0, 11 + N + T) for i, N in enumerate(Ns)]
+    x = cs[0]["x"]
+    projs = [dict(W=c["W"], bias=c["bias"], A=c["A"], B=c["B"], mask=c["mask"]) for c in cs]
+    ys, hs = mc.lora_group_forward(x, projs, 2.0, dropout_p=0.1)
+    for c, pr, y, h in zip(cs, projs, ys, hs):
+        c["x"] = x
+        y1, h1 = check_small(mc, c, c["W"], 0.1)
+        assert torch.equal(y, y1) and torch.equal(h, h1)
+    ys2, _ = mc.lora_group_forward(x, projs, 2.0, dropout_p=0.1, save_hidden=False)
+    assert all(torch.equal(a, b) for a, b in zip(ys, ys2))
+
+
 def test_lora_few_tokens_are_apart(mc, dev):
     """A non-finite token or weight row reaches its own outputs only."""
     c = small_case(dev, 5, 1032, 1000, 8, 0.0, True, 3)
