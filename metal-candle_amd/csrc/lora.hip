@@ -525,12 +525,7 @@ hipError_t launch_lora_group_fwd(const mc_lora_desc& d, const void* x, const Lor
     const LoraGroupFwdWs w = lora_group_fwd_ws(d, Ns, count);
     char* base = static_cast<char*>(ws);
     const uint16_t* xb = static_cast<const uint16_t*>(x);
-    if (few > 0) {
-        int64_t sumN = 0;
-        for (int g = 0; g < count; ++g) sumN += Ns[g];
-        auto sc = gemm_scope(st, m.T, sumN, m.K, m.r, m.r, 2);
-        return launch_lora_small_fwd(d, x, proj, count, y, h_save, base + w.small, st);
-    }
+    if (few > 0) return launch_lora_small_fwd(d, x, proj, count, y, h_save, base + w.small, st);
     uint16_t* hs = reinterpret_cast<uint16_t*>(base + w.hs_ext);
     const int ext_ld = count * m.rext;
     const int ppp = proj_per_pass(m.r);

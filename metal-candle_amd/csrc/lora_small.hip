@@ -29,6 +29,7 @@
 #include "common.hpp"
 #include "kernels.hpp"
 #include "lora_kernels.hpp"
+#include "profile.hpp"
 #include "rules.hpp"
 
 namespace mc {
@@ -297,18 +298,30 @@ hipError_t launch_lora_small_fwd(const mc_lora_desc& d, const void* x, const Lor
                             static_cast<uint16_t*>(y[g]), h_save ? h_save[g] : nullptr};
         a.tile0[g + 1] = a.tile0[g] + (proj[g].N + rows - 1) / rows;
     }
-    // h: [splits] partial sums of each projection, then one sum where they are many
-    const dim3 gh((unsigned)a.splits, (unsigned)((a.T + 15) / 16), (unsigned)count);
-    if (a.r <= 16) small_hidden<1><<<gh, 64 * kHiddenWaves<1>, 0, st>>>(a);
-    else if (a.r <= 32) small_hidden<2><<<gh, 64 * kHiddenWaves<2>, 0, st>>>(a);
-    else small_hidden<4><<<gh, 64 * kHiddenWaves<4>, 0, st>>>(a);
-    const int n = a.T * a.r;
-    if (a.splits > 1 && n * a.splits > 8192) {  // 32 KB of partial sums per workgroup of small_linear
-        float* sum = a.part + (size_t)count * a.splits * n;
-        small_hidden_sum<<<dim3((unsigned)((n + 255) / 256), (unsigned)count), 256, 0, st>>>(a.part, sum, n, a.splits);
-        a.part = sum;
-        a.splits = 1;
+    double flops = 0, bytes = 2.0 * a.T * (a.K + sumN);  // of the products; x and y
+    for (int g = 0; g < count; ++g) {
+        const double k = proj[g].W ? (double)a.K : 0.0;
+        flops += 2.0 * a.T * proj[g].N * (k > 0 ? k : a.r);
+        bytes += proj[g].N * (2.0 * k + 4.0 * a.r);
     }
+    {
+        // h: [splits] partial sums of each projection, then one sum where they are many
+        auto sc = prof::Scope(prof::kLowRank, st, 2.0 * a.T * a.K * a.r * count,
+                              2.0 * a.T * a.K + 4.0 * a.r * (a.K + a.T) * count);
+        const dim3 gh((unsigned)a.splits, (unsigned)((a.T + 15) / 16), (unsigned)count);
+        if (a.r <= 16) small_hidden<1><<<gh, 64 * kHiddenWaves<1>, 0, st>>>(a);
+        else if (a.r <= 32) small_hidden<2><<<gh, 64 * kHiddenWaves<2>, 0, st>>>(a);
+        else small_hidden<4><<<gh, 64 * kHiddenWaves<4>, 0, st>>>(a);
+        const int n = a.T * a.r;
+        if (a.splits > 1 && n * a.splits > 8192) {  // 32 KB of partial sums per workgroup of small_linear
+            float* sum = a.part + (size_t)count * a.splits * n;
+            small_hidden_sum<<<dim3((unsigned)((n + 255) / 256), (unsigned)count), 256, 0, st>>>(a.part, sum, n,
+                                                                                                 a.splits);
+            a.part = sum;
+            a.splits = 1;
+        }
+    }
+    auto sc = prof::Scope(prof::kGemm, st, flops, bytes);
     const dim3 grid((unsigned)a.tile0[count]);
     if (a.T <= 16) {
         if (wide) small_linear<1, 2, 16, 1><<<grid, 1024, 0, st>>>(a);

@@ -83,6 +83,26 @@ def test_lora_few_tokens_wide_group_equals_single(mc, dev, T, Ns, r):
     assert all(torch.equal(a, b) for a, b in zip(ys, ys2))
 
 
+def test_lora_few_tokens_are_timed_by_class(mc, dev):
+    """The timing hook books the hidden's launches as low-rank work and the
+    product with W as a GEMM, as on the tiled path."""
+    T, K, N, r = 5, 1032, 1000, 8
+    c = small_case(dev, T, K, N, r, 0.0, False, 4)
+    L = mc._lib.lib()
+    mc._lib.check(L.mc_profile_reset())
+    mc._lib.check(L.mc_profile_enable(1))
+    try:
+        mc.lora_forward(c["x"], c["A"], c["B"], 1.0, W=c["W"])
+        mc.lora_forward(c["x"], c["A"], c["B"], 1.0)
+    finally:
+        mc._lib.check(L.mc_profile_enable(0))
+    mc._lib.check(L.mc_profile_collect())
+    low, gemm = mc._lib.profile_read("lowrank"), mc._lib.profile_read("gemm")
+    mc._lib.check(L.mc_profile_reset())
+    assert low[1] == gemm[1] == 2 and low[0] > 0 and gemm[0] > 0
+    assert low[2] == 2 * (2 * T * K * r) and gemm[2] == 2 * T * N * K + 2 * T * N * r
+
+
 def test_lora_few_tokens_are_apart(mc, dev):
     """A non-finite token or weight row reaches its own outputs only."""
     c = small_case(dev, 5, 1032, 1000, 8, 0.0, True, 3)
