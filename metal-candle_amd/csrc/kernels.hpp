@@ -70,7 +70,7 @@ struct LoraGroupFwdWs {
     size_t bt_ext[kLoraMaxProj];   // per projection: bf16 [N_g][rext]
     size_t hs_ext;                 // bf16 [T][G rext]: s Hd of every projection
     size_t part;                   // split row projection: f32 [passes][splits][T][16 rc] partials of H
-    size_t small;                  // few tokens: the partial sums of H (lora_small_ws)
+    size_t small;                  // few tokens, in the place of all others: the partial sums of H (lora_small_ws)
     size_t total;
 };
 struct LoraGroupBwdWs {

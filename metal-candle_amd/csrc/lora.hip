@@ -332,8 +332,13 @@ LoraGroupFwdWs lora_group_fwd_ws(const mc_lora_desc& d, const int64_t* N, int co
         w.total = std::max(lora_group_fwd_ws(d, Ns, few).total, lora_group_fwd_ws(d, Ns + few, count - few).total);
         return w;
     }
+    if (few > 0) {
+        w.small = 0;
+        w.total = align256(lora_small_ws(m.T, m.K, m.r, count));
+        return w;
+    }
     const int ppp = proj_per_pass(m.r);
-    for (int p0 = 0, pass = 0; p0 < count; p0 += ppp, ++pass) {
+    for (int p0 = 0, pass = 0; p0 < count && !fwd_one_launch(m); p0 += ppp, ++pass) {
         const int np = count - p0 < ppp ? count - p0 : ppp;
         w.at_hilo[pass] = off;  // hi then lo, row-major [16 rc][K] or in fragment order over round_up(K, 64)
         off += align256((size_t)2 * 16 * rowproj_rc(np * m.r) * round_up(m.K, 64) * 2);
@@ -349,8 +354,6 @@ LoraGroupFwdWs lora_group_fwd_ws(const mc_lora_desc& d, const int64_t* N, int co
         const int ld = rowsplit_ld((count < ppp ? count : ppp) * m.r);
         off += align256((size_t)npass * rowsplit_splits(m.T, m.K) * m.T * ld * 4);
     }
-    w.small = off;
-    if (few > 0) off += align256(lora_small_ws(m.T, m.K, m.r, count));
     w.total = off;
     return w;
 }

@@ -69,6 +69,22 @@ def test_lora_null_and_workspace_errors(mc):
     assert "h_save" in mc._lib.last_error()
 
 
+@pytest.mark.parametrize("T,r,Ns,need", [
+    (1, 16, (1536,), 3 * 16 * 4),                    # few tokens: two partial sums of H and their sum
+    (20, 64, (1536, 256), 2 * 3 * 20 * 64 * 4),
+    (777, 16, (1536, 256), (1536 + 256) * 16 * 2 + 777 * 2 * 16 * 2),  # one launch: B^T and s Hd in bf16
+    (20, 16, (256, 8960), 8960 * 16 * 2 + 20 * 16 * 2),  # one projection of each kind: the larger
+])
+def test_lora_fwd_workspace_holds_what_its_path_writes(mc, T, r, Ns, need):
+    L = mc._lib.lib()
+    d = mc._lib.LoraDesc(T, 1536, Ns[0], r, 1.0, 0.0, 1)
+    table = (mc._lib.LoraProj * len(Ns))(*[mc._lib.LoraProj(N, None, None, 256, 256, None, None) for N in Ns])
+    got = L.mc_lora_group_fwd_workspace_size(ctypes.byref(d), table, len(Ns))
+    assert need <= got < need + 256 * 4  # each buffer rounded up to 256 bytes
+    if len(Ns) == 1:
+        assert L.mc_lora_fwd_workspace_size(ctypes.byref(d)) == got
+
+
 def test_rowop_validation(mc):
     L = mc._lib.lib()
     fake = ctypes.c_void_p(256)
