@@ -230,7 +230,8 @@ mc_status mc_softmax_bwd(int64_t rows, int64_t dim, int64_t causal_rows, int32_t
  * bf16 with D = 64 or 128 runs the MFMA (flash) kernel and needs the
  * workspace of mc_attention_fwd_workspace_size(); fp32 with
  * D % 4 == 0, D <= 128 runs on the fp32 matrix cores (a backward workspace
- * only); other D (<= 256) run a one-wave-per-row kernel. */
+ * only), from S = 5 to 16 on by D and H / Hkv; other D (<= 256) and shorter fp32
+ * sequences run a one-wave-per-row kernel. */
 typedef struct mc_attn_desc {
     int64_t batch;     /* B >= 1 */
     int64_t seq;       /* S >= 1: queries and keys (self-attention, no KV cache) */

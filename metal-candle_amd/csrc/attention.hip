@@ -31,7 +31,7 @@
 //                 log-sum-exp of every score row is saved for the backward.
 //
 // fp32 with a head dim that is a multiple of 4, at most 128: attention_f32.hip.
-// Other head dims: attn_fwd_generic, one wave per query row (lanes over the
+// Other head dims, and fp32 sequences of a few tokens: attn_fwd_generic, one wave per query row (lanes over the
 // head dim), online softmax in fp32.
 #include <algorithm>
 #include <type_traits>
@@ -1377,7 +1377,7 @@ hipError_t launch_attention_fwd(const mc_attn_desc& d, const void* q, const void
         }
         return hipGetLastError();
     }
-    if (attention_f32_mfma(d))
+    if (attention_f32_mfma_fwd(d))
         return launch_attention_f32_fwd(d, q, k, v, mask, o, lse, stream);
     const dim3 grid((unsigned)(((int64_t)B * H * S + 3) / 4));
     if (d.dtype == MC_F32)
@@ -1438,7 +1438,7 @@ AttnBwdWs attention_bwd_ws(const mc_attn_desc& d) {
         if (attention_dq_from_ds(d)) off += align256(B * H * S * (size_t)dst_ld(d.seq) * 2);
     } else {
         w.lsd = off;  off += align256(B * H * S * 4);  // Delta
-        const size_t ng = attention_f32_mfma(d) ? (size_t)attention_f32_groups(d) : 1;
+        const size_t ng = attention_f32_mfma_bwd(d) ? (size_t)attention_f32_groups(d) : 1;
         if (ng > 1) {
             w.dk_part = off;  off += align256(B * Hkv * ng * S * D * 4);
             w.dv_part = off;  off += align256(B * Hkv * ng * S * D * 4);
@@ -1515,7 +1515,7 @@ hipError_t launch_attention_bwd(const mc_attn_desc& d, const void* q, const void
         return hipGetLastError();
     }
     float* delta = reinterpret_cast<float*>(base + w.lsd);
-    if (attention_f32_mfma(d))
+    if (attention_f32_mfma_bwd(d))
         return launch_attention_f32_bwd(d, q, k, v, mask, o, lse, dout, dq, dk, dv, delta,
                                         reinterpret_cast<float*>(base + w.dk_part),
                                         reinterpret_cast<float*>(base + w.dv_part), stream);

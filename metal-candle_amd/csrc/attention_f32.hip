@@ -4,7 +4,8 @@
 // float32 tensors with a head dim that is a multiple of 4, at most 128. Every
 // product is v_mfma_f32_32x32x2_f32 (fp32 operands and sums), the softmax
 // arithmetic fp32, so the precision is that of the row-per-wave kernels these
-// replaced (attn_*_generic<float>, now only for the other head dims).
+// replaced (attn_*_generic<float>, now for the other head dims and for sequences
+// of a few tokens, attention_f32_rows_fwd / _bwd).
 //
 // What bounds it: the fp32 MFMA rate (157 TFLOP/s; a 32 x 32 block of scores
 // costs D / 2 MFMAs of 64 cycles per product), far below what LDS and L2 can
@@ -33,6 +34,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "rules.hpp"
 
 namespace mc {
 namespace {
@@ -644,8 +646,14 @@ F32AttnArgs base_args(const mc_attn_desc& d, const void* q, const void* k, const
 
 }  // namespace
 
-bool attention_f32_mfma(const mc_attn_desc& d) {
-    return d.dtype == MC_F32 && d.head_dim % 4 == 0 && d.head_dim <= 128;
+namespace {
+bool tiles_take(const mc_attn_desc& d) { return d.dtype == MC_F32 && d.head_dim % 4 == 0 && d.head_dim <= 128; }
+}  // namespace
+bool attention_f32_mfma_fwd(const mc_attn_desc& d) {
+    return tiles_take(d) && !attention_f32_rows_fwd(d.seq, d.head_dim);
+}
+bool attention_f32_mfma_bwd(const mc_attn_desc& d) {
+    return tiles_take(d) && !attention_f32_rows_bwd(d.seq, d.head_dim, d.heads / d.kv_heads);
 }
 
 int attention_f32_groups(const mc_attn_desc& d) {

@@ -144,8 +144,10 @@ hipError_t launch_attention_bwd(const mc_attn_desc& d, const void* q, const void
                                 void* dk, void* dv, void* ws, hipStream_t stream);
 
 // fp32 on the matrix cores (attention_f32.hip): head dims that are a multiple
-// of 4 (rows of whole 16-byte vectors), at most 128.
-bool attention_f32_mfma(const mc_attn_desc& d);
+// of 4 (rows of whole 16-byte vectors), at most 128, past the shortest sequences
+// (attention_f32_rows_fwd / _bwd, rules.hpp).
+bool attention_f32_mfma_fwd(const mc_attn_desc& d);
+bool attention_f32_mfma_bwd(const mc_attn_desc& d);
 // Groups that a K/V head's query heads are split into for dK/dV: the smallest
 // divisor of H / Hkv that gives 1024 workgroups (four per CU), at most one
 // head per group. A function of the shape only, as the order of the sums is.

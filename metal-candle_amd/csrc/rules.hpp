@@ -7,6 +7,19 @@
 
 namespace mc {
 
+// Float32 attention of short sequences: the row kernels (attn_*_generic, a wave
+// per row) in the place of the 32 x 32 tiles, whose work and four-wave
+// combination do not shrink with S. The row backward walks the query heads of a
+// K/V head (rep of them) one after the other. Ratio of tiles to rows, forward:
+// D 32 S 3 1.18-1.27, S 5 0.92-0.99; D 64 S 6 1.06-1.19, S 8 0.89-0.98; D 128 S 8
+// 1.07-1.19, S 10 0.94-1.05. Backward: D 32 rep 1 S 5 1.02-1.10, S 8 0.82-0.90;
+// D 64 rep 1 S 10 1.07-1.19, S 16 0.81-0.88, rep 6 S 4 0.98-1.10, S 5 0.84-0.92;
+// D 96 rep 1 S 12 1.27-1.42, D 128 rep 6 S 5 1.02-1.17, rep 7 S 6 0.77-0.94.
+constexpr bool attention_f32_rows_fwd(int64_t S, int D) { return S <= (D <= 32 ? 4 : D <= 64 ? 7 : 9); }
+constexpr bool attention_f32_rows_bwd(int64_t S, int D, int rep) {
+    return S * (rep + 2) <= (D <= 32 ? 18 : D <= 64 ? 33 : 45);
+}
+
 // Few-token LoRA forward (lora_small.hip) for one projection, else the tiled
 // path. A projection of a group takes the path that it would take alone, so
 // that the group's results are those of single calls. Up to 16 tokens it was

@@ -14,6 +14,8 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SOURCE = """
 #include "rules.hpp"
 extern "C" {
+int attention_f32_rows_fwd(int64_t S, int D) { return mc::attention_f32_rows_fwd(S, D); }
+int attention_f32_rows_bwd(int64_t S, int D, int rep) { return mc::attention_f32_rows_bwd(S, D, rep); }
 int lora_few_tokens(int64_t T, int64_t N, int r) { return mc::lora_few_tokens(T, N, r); }
 int rowproj_f32_by_token(int64_t T, int r) { return mc::rowproj_f32_by_token(T, r); }
 int colreduce_f32_tile(int64_t T, int64_t cols, int r) {
@@ -87,3 +89,22 @@ def test_rowproj_f32_by_token(rules, r, K, T, by_token, by_16):
 def test_colreduce_f32_tile(rules, r, cols, T, us):
     tile = rules.colreduce_f32_tile(ctypes.c_int64(T), ctypes.c_int64(cols), r)
     assert us[tile] <= 1.03 * min(us.values())
+
+
+# fp32 attention, time on the 32 x 32 tiles over time on the row kernels, by sequence (the worse of causal or
+# not for whichever side the rule takes; 10% either way around the crossing).
+@pytest.mark.parametrize("D,rep,fwd,bwd", [
+    (32, 1, {1: 1.73, 2: 1.38, 3: 1.18, 8: 0.74, 16: 0.45}, {1: 1.62, 2: 1.40, 3: 1.25, 10: 0.79, 16: 0.58}),
+    (64, 1, {1: 2.10, 3: 1.51, 6: 1.07, 10: 0.84, 16: 0.59}, {1: 2.21, 5: 1.49, 8: 1.20, 16: 0.88, 24: 0.70}),
+    (64, 6, {1: 2.03, 3: 1.50, 6: 1.06, 10: 0.84, 16: 0.59}, {1: 2.00, 2: 1.48, 3: 1.16, 5: 0.92, 8: 0.67}),
+    (128, 6, {1: 3.01, 4: 1.65, 8: 1.08, 12: 0.90, 24: 0.51}, {1: 2.79, 3: 1.45, 5: 1.02, 8: 0.83, 16: 0.47}),
+    (128, 7, {1: 2.81, 4: 1.65, 8: 1.07, 12: 0.90, 24: 0.27}, {1: 2.43, 3: 1.36, 4: 1.06, 6: 0.94, 8: 0.69}),
+    (96, 1, {1: 3.08, 4: 1.68, 8: 1.08, 12: 0.91, 24: 0.51}, {1: 3.57, 8: 1.62, 12: 1.27, 24: 0.89}),
+])
+def test_attention_f32_rows(rules, D, rep, fwd, bwd):
+    for S, ratio in fwd.items():
+        rows = rules.attention_f32_rows_fwd(ctypes.c_int64(S), D)
+        assert (ratio if not rows else 1 / ratio) <= 1.1, ("forward", S)
+    for S, ratio in bwd.items():
+        rows = rules.attention_f32_rows_bwd(ctypes.c_int64(S), D, rep)
+        assert (ratio if not rows else 1 / ratio) <= 1.1, ("backward", S)

@@ -29,6 +29,20 @@ def test_attention_f32_blocks(mc, dev, S, D, causal, masked):
     check_bwd(got, ref_bwd(q, k, v, mask, causal, dout), torch.float32)
 
 
+@pytest.mark.parametrize("D,S", [(32, 4), (32, 5), (32, 6), (64, 7), (64, 8), (64, 11), (64, 12), (128, 9), (128, 10),
+                                 (100, 15), (100, 16)])
+@pytest.mark.parametrize("causal,masked", [(True, False), (False, True)])
+def test_attention_f32_short(mc, dev, D, S, causal, masked):
+    """Sequences around the lengths from which the tiles take the forward and,
+    separately, the backward (whose workspace changes with them)."""
+    q, k, v, mask = case(S + D, 2, 4, 4, S, D, torch.float32, masked)
+    o, lse = run(mc, dev, q, k, v, mask, causal)
+    o_ref, lse_ref = ref(q, k, v, mask, causal)
+    check(o, lse, o_ref, lse_ref, torch.float32)
+    dout = torch.randn(2, S, 4 * D, generator=gen(S))
+    check_bwd(run_bwd(mc, dev, q, k, v, mask, causal, dout), ref_bwd(q, k, v, mask, causal, dout), torch.float32)
+
+
 @pytest.mark.parametrize("B,H,Hkv,S", [(8, 8, 4, 1000), (8, 16, 4, 500), (8, 24, 4, 400), (1, 6, 1, 100), (2, 3, 3, 70)])
 def test_attention_f32_bwd_groups(mc, dev, B, H, Hkv, S):
     """One, two, three and all query heads' partials per K/V head (the groups
