@@ -7,6 +7,22 @@
 
 namespace mc {
 
+// Softmax rows that are not whole 16-byte vectors: the covering vectors of the
+// one-wave kernels, or for short rows a lane per element (the scalar kernels),
+// where the vectors keep only a few lanes busy and pay for the shared edges.
+// us, elements / vectors, 56 heads of S x S, or 112 causal ones:
+//   fp32 forward   S 65 3.0 / 3.1 (3.8 / 4.1), S 99 3.7 / 3.5 (5.4 / 5.1), S 201 8.4 / 5.3
+//   fp32 backward  S 99 3.5 / 4.0 (5.0 / 5.7), S 161 6.5 / 5.5 (7.7 / 7.7), S 201 8.0 / 6.9
+//   bf16 forward   S 99 3.5 / 4.2 (5.0 / 6.0), S 161 6.0 / 5.4 (8.5 / 8.9), S 201 8.0 / 6.2
+//   bf16 backward  S 99 3.0 / 4.4 (4.5 / 6.2), S 201 7.0 / 6.2 (9.1 / 9.8), S 257 8.8 / 7.3
+// Enough whole rows to be bound by memory, forward, backward: 65536 rows of 77,
+// fp32 20.7 / 15.0, 21.3 / 19.0, bf16 20.4 / 21.1, 15.7 / 19.1; of 129, bf16
+// 26.6 / 21.2, 27.3 / 20.9; of 33, fp32 14.6 / 15.0, 11.1 / 17.8.
+constexpr bool softmax_ragged_vectors(int64_t rows, int64_t dim, bool causal, int elem_size, bool backward) {
+    if (rows >= 32768 && !causal) return dim >= (elem_size == 4 ? 64 : 112);
+    return dim >= (elem_size == 4 ? (backward ? 160 : 96) : (backward ? 224 : 176));
+}
+
 // Float32 attention of short sequences: the row kernels (attn_*_generic, a wave
 // per row) in the place of the 32 x 32 tiles, whose work and four-wave
 // combination do not shrink with S. The row backward walks the query heads of a

@@ -21,11 +21,13 @@
 // registers of up to 1024 threads, and rows past that (128 KB) two
 // streaming passes. Rows that are not whole 16-byte vectors run on the same
 // one-wave kernels over the aligned vectors that cover them (RowVecs), or on a
-// scalar kernel past 8 vectors per lane.
+// scalar kernel where they are short (softmax_ragged_vectors) or past 8 vectors
+// per lane.
 #include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "rules.hpp"
 
 namespace mc {
 namespace {
@@ -510,7 +512,8 @@ __global__ __launch_bounds__(kWideThreads) void softmax_bwd_stream(int64_t row0,
 
 // Row paths by length: one wave per row up to 8 vectors per lane (kWaveShared:
 // rows that are not whole 16-byte vectors, over the aligned vectors that cover
-// them; longer ones take the scalar kernels), a workgroup per row
+// them; shorter ones (softmax_ragged_vectors) and longer ones take the scalar
+// kernels), a workgroup per row
 // up to max_vpl vectors per thread of 1024 threads, else two streaming
 // passes. (One wave at 9-16 vectors per lane measured slower than the
 // workgroup per row: bf16 [8192, 8192] backward 137 against 61 us, forward
@@ -526,8 +529,11 @@ int64_t row_vectors(int64_t dim) {
 }
 
 template <typename T>
-RowPath row_path(int64_t dim, int max_vpl) {
-    if (dim % Vec16<T>::N != 0) return row_vectors<T>(dim) <= 8 * kWave ? RowPath::kWaveShared : RowPath::kScalar;
+RowPath row_path(int64_t rows, int64_t dim, int64_t causal, int max_vpl, bool backward) {
+    if (dim % Vec16<T>::N != 0)
+        return row_vectors<T>(dim) <= 8 * kWave && softmax_ragged_vectors(rows, dim, causal > 0, (int)sizeof(T), backward)
+                   ? RowPath::kWaveShared
+                   : RowPath::kScalar;
     const int64_t nvec = dim / Vec16<T>::N;
     if (nvec <= 8 * kWave) return RowPath::kWave;
     if (nvec <= (int64_t)max_vpl * kWideThreads) return RowPath::kWide;
@@ -572,7 +578,7 @@ template <typename T>
 hipError_t fwd_impl(int64_t rows, int64_t dim, int64_t causal, const void* s, void* p, hipStream_t st) {
     const T* sp = static_cast<const T*>(s);
     T* pp = static_cast<T*>(p);
-    const RowPath path = row_path<T>(dim, 8);
+    const RowPath path = row_path<T>(rows, dim, causal, 8, false);
     if (path == RowPath::kWide) {
         const WideShape w = wide_shape<T>(dim);
         const int d = (int)dim;
@@ -612,7 +618,7 @@ hipError_t bwd_impl(int64_t rows, int64_t dim, int64_t causal, const void* p, co
     const T* pp = static_cast<const T*>(p);
     const T* gp = static_cast<const T*>(dp);
     T* dsp = static_cast<T*>(ds);
-    const RowPath path = row_path<T>(dim, sizeof(T) == 2 ? 4 : 8);
+    const RowPath path = row_path<T>(rows, dim, causal, sizeof(T) == 2 ? 4 : 8, true);
     if (path == RowPath::kWide) {
         const WideShape w = wide_shape<T>(dim);
         const int d = (int)dim;

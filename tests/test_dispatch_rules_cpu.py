@@ -14,6 +14,9 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SOURCE = """
 #include "rules.hpp"
 extern "C" {
+int softmax_ragged_vectors(int64_t rows, int64_t dim, int causal, int elem_size, int backward) {
+    return mc::softmax_ragged_vectors(rows, dim, causal != 0, elem_size, backward != 0);
+}
 int attention_f32_rows_fwd(int64_t S, int D) { return mc::attention_f32_rows_fwd(S, D); }
 int attention_f32_rows_bwd(int64_t S, int D, int rep) { return mc::attention_f32_rows_bwd(S, D, rep); }
 int lora_few_tokens(int64_t T, int64_t N, int r) { return mc::lora_few_tokens(T, N, r); }
@@ -108,3 +111,31 @@ def test_attention_f32_rows(rules, D, rep, fwd, bwd):
     for S, ratio in bwd.items():
         rows = rules.attention_f32_rows_bwd(ctypes.c_int64(S), D, rep)
         assert (ratio if not rows else 1 / ratio) <= 1.1, ("backward", S)
+
+
+# Softmax rows of S elements, 56 heads of S x S and 112 causal ones, us: (elements, covering vectors) of each.
+@pytest.mark.parametrize("size,backward,S,plain,causal", [
+    (4, 0, 9, (2.3, 2.6), (2.4, 2.7)), (4, 0, 33, (2.4, 2.8), (2.8, 3.3)), (4, 0, 65, (3.0, 3.1), (3.8, 4.1)),
+    (4, 0, 99, (3.7, 3.5), (5.4, 5.1)), (4, 0, 201, (8.4, 5.3), (11.7, 8.2)), (4, 0, 777, (113.0, 44.1), (176.8, 75.3)),
+    (4, 1, 33, (2.2, 2.8), (2.4, 3.5)), (4, 1, 99, (3.5, 4.0), (5.0, 5.7)), (4, 1, 161, (6.5, 5.5), (7.7, 7.7)),
+    (4, 1, 301, (17.6, 13.5), (24.8, 19.4)), (4, 1, 777, (122.4, 76.8), (148.1, 111.0)),
+    (2, 0, 33, (2.4, 3.1), (2.9, 3.8)), (2, 0, 99, (3.5, 4.2), (5.0, 6.0)), (2, 0, 201, (8.0, 6.2), (11.0, 10.2)),
+    (2, 0, 777, (92.8, 32.4), (120.0, 54.9)), (2, 1, 33, (2.2, 3.1), (2.4, 3.8)), (2, 1, 77, (2.7, 4.0), (3.7, 5.5)),
+    (2, 1, 129, (4.0, 4.9), (5.9, 7.5)), (2, 1, 257, (8.8, 7.3), (12.5, 11.6)), (2, 1, 1023, (132.7, 101.8), (192.2, 189.7)),
+])
+def test_softmax_ragged_vectors(rules, size, backward, S, plain, causal):
+    for heads, c, us in ((56, 0, plain), (112, 1, causal)):
+        vectors = rules.softmax_ragged_vectors(ctypes.c_int64(heads * S), ctypes.c_int64(S), c, size, backward)
+        assert us[vectors] <= 1.03 * min(us)
+
+
+# 65536 rows, no mask.
+@pytest.mark.parametrize("size,dim,forward,backward", [
+    (4, 33, (14.6, 15.0), (11.1, 17.8)), (4, 77, (20.7, 15.0), (21.3, 19.0)), (4, 129, (30.9, 16.8), (31.1, 27.4)),
+    (2, 33, (14.2, 21.3), (10.8, 19.2)), (2, 77, (20.4, 21.1), (15.7, 19.1)), (2, 129, (26.6, 21.2), (27.3, 20.9)),
+    (2, 301, (52.1, 23.6), (47.8, 29.9)),
+])
+def test_softmax_ragged_vectors_many_rows(rules, size, dim, forward, backward):
+    for b, us in enumerate((forward, backward)):
+        vectors = rules.softmax_ragged_vectors(ctypes.c_int64(65536), ctypes.c_int64(dim), 0, size, b)
+        assert us[vectors] == min(us)
