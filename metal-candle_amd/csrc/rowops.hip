@@ -21,12 +21,13 @@
 // Vocabulary rows are long (10^5 entries), so these use one workgroup (256 or
 // 1024 threads) per row with an online (max, sum) per thread, combined in a
 // fixed order. The loss is a second, single-workgroup pass over the per-row
-// values in row order, so it is bitwise reproducible.
+// values in a fixed order, so it is bitwise reproducible.
 #include <type_traits>
 
 #include "column_sum.hpp"
 #include "common.hpp"
 #include "kernels.hpp"
+#include "rules.hpp"
 
 namespace mc {
 namespace {
@@ -1079,13 +1080,8 @@ hipError_t launch_log_softmax_bwd(int64_t rows, int64_t dim, int dtype, const vo
     return hipGetLastError();
 }
 
-// Threads per row of the cross-entropy passes: 256, which keeps 8 rows on a CU
-// for the loads in flight; 1024 where fewer rows than that would leave the CUs
-// short of them and a row has work for all (forward and backward of 64 bf16
-// rows of 151936: 76 -> 36 us; 500 of 8001: 31 -> 16 us).
-bool xent_wide(const mc_xent_desc& d) {
-    return d.rows < 1024 && d.vocab >= 1024 * (d.dtype == MC_F32 ? 4 : 8);
-}
+// Threads per row of the cross-entropy passes (the same in both).
+bool xent_wide(const mc_xent_desc& d) { return xent_wide_rows(d.rows, d.vocab, d.dtype == MC_F32 ? 4 : 2); }
 
 hipError_t launch_cross_entropy_fwd(const mc_xent_desc& d, const void* logits, const uint32_t* targets, float* loss,
                                     float* stats, float* ws, hipStream_t stream) {

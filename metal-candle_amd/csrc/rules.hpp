@@ -7,6 +7,19 @@
 
 namespace mc {
 
+// Cross-entropy rows on 1024 threads instead of 256, where so few rows leave
+// CUs short of loads in flight and a row has work for all the threads. Forward and backward,
+// us, 1024 / 256 threads:
+//   rows 64    fp32 8001 14.0 / 15.9, 50257 21.7 / 40.5; bf16 8192 12.9 / 11.7, 32000 18.6 / 23.0
+//   rows 256   fp32 8192 15.3 / 15.7, 32000 25.8 / 30.3; bf16 16384 16.0 / 16.6, 151936 50.5 / 78.0
+//   rows 384   fp32 8192 19.0 / 16.3, 32000 36.8 / 40.2; bf16 16384 19.7 / 17.9, 50257 34.8 / 36.3
+//   rows 512   fp32 16384 27.6 / 24.7, 50257 63.3 / 64.9; bf16 32000 29.4 / 27.7, 151936 95.3 / 116
+//   rows 1000  fp32 8192 30.5 / 23.9, 151936 333 / 333; bf16 8192 26.4 / 19.1, 50257 66.3 / 62.8
+constexpr bool xent_wide_rows(int64_t rows, int64_t vocab, int elem_size) {
+    const int64_t vectors = vocab * elem_size / 16;
+    return rows <= 256 ? vectors >= 1536 : rows <= 512 && vectors >= 6144;
+}
+
 // Softmax rows that are not whole 16-byte vectors: the covering vectors of the
 // one-wave kernels, or for short rows a lane per element (the scalar kernels),
 // where the vectors keep only a few lanes busy and pay for the shared edges.

@@ -14,6 +14,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SOURCE = """
 #include "rules.hpp"
 extern "C" {
+int xent_wide_rows(int64_t rows, int64_t vocab, int elem_size) { return mc::xent_wide_rows(rows, vocab, elem_size); }
 int softmax_ragged_vectors(int64_t rows, int64_t dim, int causal, int elem_size, int backward) {
     return mc::softmax_ragged_vectors(rows, dim, causal != 0, elem_size, backward != 0);
 }
@@ -139,3 +140,24 @@ def test_softmax_ragged_vectors_many_rows(rules, size, dim, forward, backward):
     for b, us in enumerate((forward, backward)):
         vectors = rules.softmax_ragged_vectors(ctypes.c_int64(65536), ctypes.c_int64(dim), 0, size, b)
         assert us[vectors] == min(us)
+
+
+# Cross-entropy forward and backward, us: 256 threads, 1024 threads, by rows.
+@pytest.mark.parametrize("size,V,us", [
+    (4, 4096, {64: (11.4, 12.5), 512: (14.2, 17.3), 1000: (17.5, 25.2)}),
+    (4, 8001, {64: (15.9, 14.0), 200: (16.7, 15.4)}),
+    (2, 10001, {64: (13.1, 13.5), 128: (14.7, 14.5)}),
+    (4, 8192, {64: (13.8, 13.6), 256: (15.7, 15.3), 384: (16.3, 19.0), 640: (19.1, 24.9), 1000: (23.9, 30.5)}),
+    (4, 16384, {128: (19.6, 16.7), 256: (20.4, 19.2), 384: (22.4, 24.4), 512: (24.7, 27.6)}),
+    (4, 32000, {64: (28.5, 18.7), 256: (30.3, 25.8), 384: (40.2, 36.8), 640: (52.9, 54.7)}),
+    (4, 151936, {64: (110.8, 44.5), 384: (165.7, 132.4), 512: (183.3, 165.2), 1023: (339.8, 338.8)}),
+    (2, 8192, {64: (11.7, 12.9), 256: (13.6, 14.2), 512: (15.3, 18.0), 1000: (19.1, 26.4)}),
+    (2, 16384, {64: (15.3, 15.0), 256: (16.6, 16.0), 384: (17.9, 19.7), 1000: (25.4, 32.2)}),
+    (2, 32000, {128: (22.8, 19.5), 256: (23.8, 21.1), 512: (27.7, 29.4), 1000: (44.6, 50.4)}),
+    (2, 50257, {64: (28.6, 20.6), 384: (36.3, 34.8), 512: (41.3, 39.9), 768: (51.9, 53.9)}),
+    (2, 151936, {64: (63.7, 35.9), 512: (115.6, 95.3), 768: (134.8, 131.3), 896: (153.1, 154.6)}),
+])
+def test_xent_wide_rows(rules, size, V, us):
+    for rows, t in us.items():
+        wide = rules.xent_wide_rows(ctypes.c_int64(rows), ctypes.c_int64(V), size)
+        assert t[wide] <= 1.04 * min(t), rows
