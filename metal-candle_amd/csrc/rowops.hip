@@ -631,15 +631,17 @@ __device__ __forceinline__ void store_nt16(uint16_t* p, const float (&v)[8]) {
 
 // dlogits = dloss ((1 - s) valid (p - onehot(t)) / count + s (p - 1/V) / rows), p = exp(x - lse)
 // vec: the rows of logits and dlogits start alike inside a 16-byte vector.
+// stream: dlogits are stored past the caches (xent_stream_gradients).
 // Bound by HBM. The pass usually follows the forward's over the same logits,
 // whose last columns of the last rows are then in the 256 MB last-level cache:
-// rows and columns run backwards to meet them, and dlogits are stored
-// non-temporally so as not to push them out. Forward and backward of 2036 bf16
-// rows of 151936: 395 us in forward order with write-back stores, 382 reversed,
-// 342 with both; 1500 fp32 rows of 50257: 195 reversed, 158 with both.
+// rows and columns run backwards to meet them. Forward and backward, logits not
+// seen before the forward: 2036 bf16 rows of 151936 401 us in forward order, 384
+// reversed, 333 reversed and streamed; 1500 fp32 rows of 50257 196 reversed, 161
+// streamed. With more logits than a few times the cache the order gains
+// nothing (16384 bf16 rows of 151936: 2.8 ms either way).
 template <typename T, int NT>
-__global__ __launch_bounds__(NT) void xent_bwd_k(int64_t rows, int64_t vocab, bool vec, float smoothing,
-                                                 const T* __restrict__ logits, const uint32_t* __restrict__ targets,
+__global__ __launch_bounds__(NT) void xent_bwd_k(int64_t rows, int64_t vocab, bool vec, bool stream,
+                                                 float smoothing, const T* __restrict__ logits, const uint32_t* __restrict__ targets,
                                                  int64_t ignore_index, const float* __restrict__ stats,
                                                  const float* __restrict__ dloss, T* __restrict__ dlogits) {
     constexpr int N = Vec16<T>::N;
@@ -666,7 +668,8 @@ __global__ __launch_bounds__(NT) void xent_bwd_k(int64_t rows, int64_t vocab, bo
             Vec16<T>::load(xr + j0, v);
 #pragma unroll
             for (int e = 0; e < N; ++e) v[e] = grad(v[e], j0 + e);
-            store_nt16(dr + j0, v);
+            if (stream) store_nt16(dr + j0, v);
+            else Vec16<T>::store(dr + j0, v);
         }
         const int64_t j = span.edge((int)threadIdx.x, vocab);
         if (j >= 0) Elem<T>::store(dr, j, grad(Elem<T>::load(xr, j), j));
@@ -1111,8 +1114,10 @@ hipError_t launch_cross_entropy_bwd(const mc_xent_desc& d, const void* logits, c
     auto go = [&](auto elem, auto threads) {
         typedef decltype(elem) T;
         constexpr int NT = decltype(threads)::value;
-        xent_bwd_k<T, NT><<<grid, NT, 0, stream>>>(d.rows, d.vocab, vec, d.smoothing, static_cast<const T*>(logits),
-                                                   targets, d.ignore_index, stats, dloss, static_cast<T*>(dlogits));
+        xent_bwd_k<T, NT><<<grid, NT, 0, stream>>>(d.rows, d.vocab, vec,
+                                                   xent_stream_gradients(d.rows, d.vocab, sizeof(T)), d.smoothing,
+                                                   static_cast<const T*>(logits), targets, d.ignore_index, stats,
+                                                   dloss, static_cast<T*>(dlogits));
     };
     auto by_dtype = [&](auto threads) {
         if (d.dtype == MC_F32) go(float{}, threads);

@@ -14,6 +14,9 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SOURCE = """
 #include "rules.hpp"
 extern "C" {
+int xent_stream_gradients(int64_t rows, int64_t vocab, int elem_size) {
+    return mc::xent_stream_gradients(rows, vocab, elem_size);
+}
 int xent_wide_rows(int64_t rows, int64_t vocab, int elem_size) { return mc::xent_wide_rows(rows, vocab, elem_size); }
 int softmax_ragged_vectors(int64_t rows, int64_t dim, int causal, int elem_size, int backward) {
     return mc::softmax_ragged_vectors(rows, dim, causal != 0, elem_size, backward != 0);
@@ -161,3 +164,24 @@ def test_xent_wide_rows(rules, size, V, us):
     for rows, t in us.items():
         wide = rules.xent_wide_rows(ctypes.c_int64(rows), ctypes.c_int64(V), size)
         assert t[wide] <= 1.04 * min(t), rows
+
+
+# Cross-entropy forward and backward alone, and followed by a pass over the gradients, on logits not seen before,
+# us: ordinary stores, streamed.
+@pytest.mark.parametrize("size,rows,V,alone,followed", [
+    (4, 497, 50257, (63.3, 62.6), (92.2, 96.7)), (4, 781, 32000, (69.8, 64.6), (98.3, 100.5)),
+    (4, 164, 151936, (69.6, 62.6), (90.5, 91.5)), (4, 1093, 32000, (96.0, 82.2), (138.6, 128.7)),
+    (4, 795, 50257, (109.7, 99.0), (164.1, 150.6)), (4, 1492, 50257, (186.8, 157.6), (281.0, 265.5)),
+    (2, 994, 50257, (67.8, 65.5), (96.4, 100.2)), (2, 1562, 32000, (70.7, 65.1), (95.7, 100.7)),
+    (2, 460, 151936, (100.1, 88.3), (142.8, 128.7)), (2, 1989, 50257, (138.7, 119.6), (196.9, 187.4)),
+    (2, 2036, 151936, (384.4, 333.1), (577.3, 561.6)),
+])
+def test_xent_stream_gradients(rules, size, rows, V, alone, followed):
+    stream = rules.xent_stream_gradients(ctypes.c_int64(rows), ctypes.c_int64(V), size)
+    assert followed[stream] == min(followed)
+    assert alone[stream] <= 1.12 * min(alone)
+
+
+def test_xent_stream_gradients_line(rules):
+    assert not rules.xent_stream_gradients(ctypes.c_int64(96 << 10), ctypes.c_int64(512), 2)
+    assert rules.xent_stream_gradients(ctypes.c_int64((96 << 10) + 1), ctypes.c_int64(512), 2)
