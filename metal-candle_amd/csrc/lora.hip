@@ -141,13 +141,17 @@ int few_first(const Dims& m, const int64_t* N, int count, int (&sel)[kMaxProj]) 
 // The forward's preparation and row projection as one launch
 // (launch_lora_fwd_operands). It reads x once per projection and repeats A's
 // strided reads for every 16 tokens, so it wins while launches and the wait
-// between them are the larger part. Forward, two launches -> one: K 1536,
-// N 8960, T 777 40.7 -> 34.5 us; K 3584, N 512, T 1243 42.5 -> 33.2; K 1536,
-// N 256, T 2048 23.7 -> 17.6; K 3584, N 512, r 32, T 4096 54.1 -> 51.0; three
-// projections of K 3584, T 4096 even. Past that it loses (forward and backward,
-// T 8000: K 1536, N 1536 / 256 / 256 155 -> 165 us), and where the split row
-// projection runs it is not taken. The line is on T, K and r only, so a group
-// computes what its projections would alone.
+// between them are the larger part. Forward, two launches -> one, us: K 1536,
+// N 8960, T 777 46 -> 34; K 1536, N 1536, r 8, T 4096 36.6 -> 32.4; K 896, N 896,
+// r 8, T 4000 23.4 -> 18.5; N 1536 / 256 / 256, r 8, T 2048 32.8 -> 29.3. Past
+// 4096 it loses (forward and backward, T 8000: K 1536, N 1536 / 256 / 256 155 ->
+// 165), and where the split row projection runs it is not taken. Groups of
+// three and four small projections, whose two launches read x once for all,
+// cross earlier: N 1536 / 256 / 256, r 8, T 3000 38.3 -> 39.0, T 4096 41.5 ->
+// 43.9, four of N 256, T 4096 32.4 -> 37.8. The line is on T, K and r only all
+// the same, so that a group computes what its projections would alone; two
+// projections of 16 ranks per workgroup from one read of x did not move it (T
+// 4096 44.9).
 constexpr int64_t kFwdOneTokens = 4096;
 bool fwd_one_launch(const Dims& m) { return m.r <= kFwdOpRanks && m.T <= kFwdOneTokens && !fwd_rowsplit(m); }
 

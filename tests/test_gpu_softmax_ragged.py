@@ -4,7 +4,9 @@ start of a row inside a vector, the shortest and longest such rows, and the
 scalar kernels on both sides of them.
 
 Against the oracle, tolerances as in test_gpu_rowops.py (fp32 1e-5, bf16 2e-2
-of the largest value).
+of the largest value), and each element against float64: 1e-5 of its terms (the
+exponential of an fp32 difference of at most 27: 2e-6, and the fp32 sums), plus,
+in bf16, the rounding of the result, 2^-8 of it.
 """
 import pytest
 import torch
@@ -18,9 +20,29 @@ DIMS = {torch.float32: [1, 2, 3, 5, 7, 63, 65, 95, 97, 98, 99, 159, 161, 253, 25
         torch.bfloat16: [1, 3, 7, 9, 12, 63, 65, 175, 177, 223, 225, 226, 227, 228, 229, 230, 231, 509, 513, 777, 1023, 4082, 4083, 4089]}
 
 
+def check_elements(got, want, terms, dtype):
+    bound = 1e-5 * terms + (0.0 if dtype == torch.float32 else 2.0 ** -8) * want.abs()
+    bad = ~((got.double() - want).abs() <= bound)  # a NaN, too
+    assert not bad.any(), f"{int(bad.sum())} elements, the first at {bad.nonzero()[0].tolist()}"
+
+
+def check_exact(s, p, dp, ds, S, dtype):
+    """p against the softmax of s, ds against its gradient at p, whole tensors."""
+    rows, dim = s.shape
+    x = s.double()
+    if S:
+        lim = torch.arange(rows, device=s.device)[:, None] % S + (dim - S)
+        x = x.masked_fill(torch.arange(dim, device=s.device)[None, :] > lim, float("-inf"))
+    want = torch.softmax(x, -1)
+    check_elements(p, want, want, dtype)
+    q, g = p.double(), dp.double()
+    terms = q * (g.abs() + (q * g).abs().sum(-1, keepdim=True))
+    check_elements(ds, q * (g - (q * g).sum(-1, keepdim=True)), terms, dtype)
+
+
 @pytest.mark.parametrize("dtype,dim", [(t, d) for t, ds in DIMS.items() for d in ds])
 @pytest.mark.parametrize("causal", [False, True])
-def test_softmax_ragged_rows(mc, dev, dtype, dim, causal):
+def test_softmax_ragged_rows(mc, dev, nan_outputs, dtype, dim, causal):
     g = torch.Generator().manual_seed(dim)
     rows = 11 if dim > 300 else 37
     S = min(dim, 6) if causal else 0
@@ -33,6 +55,7 @@ def test_softmax_ragged_rows(mc, dev, dtype, dim, causal):
     ds = mc.softmax_backward(p, dp.to(dev), S)
     ds_ref = oracle.softmax_bwd(p.float().cpu().numpy(), dp.float().numpy(), causal_rows=S)
     assert rel_err(ds, ds_ref) <= tol
+    check_exact(s.to(dev), p, dp.to(dev), ds, S, dtype)
     if causal:
         keep = torch.arange(dim)[None, :] <= (torch.arange(rows) % S)[:, None] + (dim - S)
         assert not p.cpu()[~keep].any() and not ds.cpu()[~keep].any()
@@ -41,19 +64,14 @@ def test_softmax_ragged_rows(mc, dev, dtype, dim, causal):
 @pytest.mark.parametrize("dtype,dim", [(torch.float32, 63), (torch.float32, 65), (torch.bfloat16, 111),
                                        (torch.bfloat16, 113)])
 @pytest.mark.parametrize("rows", [32767, 32769])
-def test_softmax_ragged_many_rows(mc, dev, dtype, dim, rows):
+def test_softmax_ragged_many_rows(mc, dev, nan_outputs, dtype, dim, rows):
     """Both sides of the rule for many unmasked rows, whole tensors."""
     g = torch.Generator(device=dev).manual_seed(dim)
     s = (torch.randn(rows, dim, generator=g, device=dev) * 3).to(dtype)
     dp = torch.randn(rows, dim, generator=g, device=dev).to(dtype)
     p = mc.softmax_forward(s)
     ds = mc.softmax_backward(p, dp)
-    want = torch.softmax(s.double(), -1)
-    q = p.double()
-    wds = q * (dp.double() - (q * dp.double()).sum(-1, keepdim=True))
-    tol = 1e-5 if dtype == torch.float32 else 2e-2
-    assert float((q - want).abs().max()) <= tol * float(want.max())
-    assert float((ds.double() - wds).abs().max()) <= tol * float(wds.abs().max())
+    check_exact(s, p, dp, ds, 0, dtype)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
