@@ -290,6 +290,18 @@ __device__ __forceinline__ void wait_vmcnt() {
 // Wave index within the workgroup as a scalar (wave-uniform) value.
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
+// v(0) + ... + v(n - 1), four at a time, in a fixed order.
+template <typename F>
+__device__ __forceinline__ float sum_tree(int n, F&& v) {
+    float t = 0.f;
+    for (int w = 0; w < n; w += 4) {
+        const float a = v(w) + (w + 1 < n ? v(w + 1) : 0.f);
+        const float b = (w + 2 < n ? v(w + 2) : 0.f) + (w + 3 < n ? v(w + 3) : 0.f);
+        t = w == 0 ? a + b : t + (a + b);
+    }
+    return t;
+}
+
 // ------------------------------------------------- workgroup reductions
 // Over every wave of a workgroup of up to kMaxWaves waves: each wave's
 // butterfly result goes to red[wave]; after the barrier every thread combines

@@ -300,7 +300,7 @@ struct GemmPlan {
 GemmPlan choose_gemm_plan(int64_t M, int64_t N, int64_t K, int cus);
 
 // ------------------------------------------------------------- fp32 path
-// Same contracts as above with fp32 storage and plain FMA arithmetic; used
+// Same contracts as above with fp32 storage, on the fp32 matrix cores; used
 // for act_dtype == MC_F32 (the fp32 parity configuration).
 struct GemmSegF32 {
     const float* a;

@@ -27,7 +27,8 @@
 //  the out-of-range rows and columns, so their loops have no branches and
 //  issue every load of an unrolled block before its MFMAs.
 //
-// fp32 variants (plain FMA) serve act_dtype == MC_F32.
+// fp32 variants (rowproj_f32, colreduce_f32, on the fp32 matrix cores) serve
+// act_dtype == MC_F32.
 #include <algorithm>
 #include <type_traits>
 
@@ -1323,18 +1324,6 @@ __device__ __forceinline__ f32x4 load4_n(const float* p, int64_t n) {
     return v;
 }
 
-// Sum of the waves' values v(0) .. v(nw - 1): four at a time, in a fixed order.
-template <typename F>
-__device__ __forceinline__ float wave_tree(int nw, F&& v) {
-    float t = 0.f;
-    for (int w = 0; w < nw; w += 4) {
-        const float a = v(w) + (w + 1 < nw ? v(w + 1) : 0.f);
-        const float b = (w + 2 < nw ? v(w + 2) : 0.f) + (w + 3 < nw ? v(w + 3) : 0.f);
-        t = w == 0 ? a + b : t + (a + b);
-    }
-    return t;
-}
-
 // fp32 row projection v[t][j] = sum_c X[t][c] P(j, c) on v_mfma_f32_16x16x4_f32:
 // a workgroup owns 16 tokens and 16 RT ranks, its waves take every nw-th block
 // of 32 NB columns. Lane l supplies token (rank) l % 16 and, for MFMA q of a
@@ -1436,7 +1425,7 @@ __global__ __launch_bounds__(64 * kF32RowWaves<RT>) void rowproj_f32(const float
         const int rt = o >> 8, tl = o & 15, jl = (o >> 4) & 15, j = j0 + 16 * rt + jl;
         const int64_t t = t0 + tl;
         if (t >= T || j >= r) continue;
-        float v = scale * wave_tree(nw, [&](int w) { return red[w][rt][tl][jl]; });
+        float v = scale * sum_tree(nw, [&](int w) { return red[w][rt][tl][jl]; });
         if (mask) v = mask[t * r + j] ? v * keep : 0.f;
         if (out_t) out_t[(int64_t)j * T + t] = v;
         if (out_ext) out_ext[t * r + j] = v * ext_scale;
@@ -1584,7 +1573,7 @@ __global__ __launch_bounds__(64 * kFwdOpWaves) void lora_fwd_operands(FwdOperand
         if (t >= T || j >= b.rext) continue;
         float v = 0.f;
         if (j < r) {
-            v = wave_tree(kFwdOpWaves, [&](int w) { return red[w][rt][tl][jl]; });
+            v = sum_tree(kFwdOpWaves, [&](int w) { return red[w][rt][tl][jl]; });
             if (P.mask) v = P.mask[t * r + j] ? v * b.keep : 0.f;
             if (P.h_save) P.h_save[(int64_t)j * T + t] = v;
         }
@@ -1705,7 +1694,7 @@ __global__ __launch_bounds__(64 * kF32ColWaves<RT>) void colreduce_f32(int64_t T
             const int j = j0 + 16 * rt + jl;
             const int64_t c = c0 + cl;
             if (j >= r || c >= C) continue;
-            const float v = J.scale * wave_tree(nw, [&](int w) { return red[w][jl][cl]; });
+            const float v = J.scale * sum_tree(nw, [&](int w) { return red[w][jl][cl]; });
             if (J.transpose_out) J.out[c * r + j] = v;
             else J.out[(int64_t)j * C + c] = v;
         }

@@ -55,18 +55,6 @@ struct SmallArgs {
     float scale, keep;
 };
 
-// a + b + ... over 0 .. n - 1, four at a time, in a fixed order
-template <typename F>
-__device__ __forceinline__ float sum_tree(int n, F&& v) {
-    float t = 0.f;
-    for (int w = 0; w < n; w += 4) {
-        const float a = v(w) + (w + 1 < n ? v(w + 1) : 0.f);
-        const float b = (w + 2 < n ? v(w + 2) : 0.f) + (w + 3 < n ? v(w + 3) : 0.f);
-        t = w == 0 ? a + b : t + (a + b);
-    }
-    return t;
-}
-
 // Grid (splits, 16-token tiles, projections). Lane l supplies token (rank)
 // l % 16 and, for MFMA q of a 16-column group, column 4 (l / 16) + q; a wave
 // takes every nw-th block of 32 columns of the split.
