@@ -88,7 +88,8 @@ mc_status check_lora_desc(const mc_lora_desc* d) {
 
 // One launch holds at most 2^32 - 1 work-items. The RMSNorm and LayerNorm
 // forward kernels run one 64-lane wave per row, four rows per 256-thread
-// workgroup; log_softmax and cross-entropy one 256-thread workgroup per row.
+// workgroup; log_softmax and cross-entropy one 256-thread workgroup per row
+// (cross-entropy 1024 threads only where rows are at most 512).
 // (Softmax splits its launches by rows and has no such bound.)
 constexpr int64_t kMaxWaveRows = ((((int64_t)1 << 32) - 1) / 256) * 4;  // 67108860
 constexpr int64_t kMaxBlockRows = (((int64_t)1 << 32) - 1) / 256;       // 16777215

@@ -502,7 +502,8 @@ __global__ __launch_bounds__(256, kWgPerCu<DP>) void attn_f32_bwd_dq(F32AttnArgs
 // -------------------------------------------------------------------- dK, dV
 // One workgroup per (b, K/V head, group of query heads, 32 keys): the waves
 // take every 4th (head, query block) of the group. K stays in registers and V
-// in an LDS tile that the waves share (both in registers spilled at D = 64);
+// in an LDS tile that the waves share (at D = 64 this form spills 16 VGPRs, 24
+// with a mask, and both in registers spilled more);
 // Q and dO rows go through the wave's LDS tiles and are read both ways:
 // S = Q.K^T, dP = dO.V^T (lane = key, registers = queries), dV^T += dO^T.P,
 // dK^T += Q^T.dS.
@@ -647,7 +648,10 @@ F32AttnArgs base_args(const mc_attn_desc& d, const void* q, const void* k, const
 }  // namespace
 
 namespace {
-bool tiles_take(const mc_attn_desc& d) { return d.dtype == MC_F32 && d.head_dim % 4 == 0 && d.head_dim <= 128; }
+bool tiles_take(const mc_attn_desc& d) {
+    return d.dtype == MC_F32 && d.head_dim % 4 == 0 && d.head_dim <= 128 &&
+           attention_f32_tiles_fit(d.seq, d.batch * d.heads);
+}
 }  // namespace
 bool attention_f32_mfma_fwd(const mc_attn_desc& d) {
     return tiles_take(d) && !attention_f32_rows_fwd(d.seq, d.head_dim);

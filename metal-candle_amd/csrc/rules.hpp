@@ -67,6 +67,12 @@ constexpr bool attention_f32_rows_bwd(int64_t S, int D, int rep) {
     return S * (rep + 2) <= (D <= 32 ? 18 : D <= 64 ? 33 : 45);
 }
 
+// The tiles' launches, 256 threads per 32 rows of a head, stay within 2^32 - 1
+// work-items (the row kernels take 64 per row, fewer where S is 1 to 3).
+constexpr bool attention_f32_tiles_fit(int64_t S, int64_t batch_heads) {
+    return (S + 31) / 32 * batch_heads <= (((int64_t)1 << 32) - 1) / 256;
+}
+
 // Few-token LoRA forward (lora_small.hip) for one projection, else the tiled
 // path. A projection of a group takes the path that it would take alone, so
 // that the group's results are those of single calls. Up to 16 tokens it was

@@ -21,6 +21,7 @@ int xent_wide_rows(int64_t rows, int64_t vocab, int elem_size) { return mc::xent
 int softmax_ragged_vectors(int64_t rows, int64_t dim, int causal, int elem_size, int backward) {
     return mc::softmax_ragged_vectors(rows, dim, causal != 0, elem_size, backward != 0);
 }
+int attention_f32_tiles_fit(int64_t S, int64_t bh) { return mc::attention_f32_tiles_fit(S, bh); }
 int attention_f32_rows_fwd(int64_t S, int D) { return mc::attention_f32_rows_fwd(S, D); }
 int attention_f32_rows_bwd(int64_t S, int D, int rep) { return mc::attention_f32_rows_bwd(S, D, rep); }
 int lora_few_tokens(int64_t T, int64_t N, int r) { return mc::lora_few_tokens(T, N, r); }
@@ -185,3 +186,12 @@ def test_xent_stream_gradients(rules, size, rows, V, alone, followed):
 def test_xent_stream_gradients_line(rules):
     assert not rules.xent_stream_gradients(ctypes.c_int64(96 << 10), ctypes.c_int64(512), 2)
     assert rules.xent_stream_gradients(ctypes.c_int64((96 << 10) + 1), ctypes.c_int64(512), 2)
+
+
+def test_attention_f32_tiles_fit(rules):
+    """One launch holds at most 2^32 - 1 work-items; calls that the tiles would
+    take past that stay with the row kernels."""
+    for S, bh, want in ((2, 16777215, 1), (2, 16777216, 0), (33, 8388607, 1), (33, 8388608, 0), (1 << 20, 511, 1)):
+        assert rules.attention_f32_tiles_fit(ctypes.c_int64(S), ctypes.c_int64(bh)) == want
+        if want:
+            assert (S + 31) // 32 * bh * 256 < 1 << 32
