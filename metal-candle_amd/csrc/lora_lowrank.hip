@@ -1330,8 +1330,8 @@ __device__ __forceinline__ f32x4 load4_n(const float* p, int64_t n) {
 // 16-column group, column 4 (l / 16) + q, so a lane loads 16 bytes of its row
 // of x and four lanes a 64-byte segment; the next block is requested before a
 // block is multiplied. Bound by the reads of x: the one workgroup per token
-// that it replaces read all of P for each token (2036 x 8960, r 16: 280 -> 51
-// us; 2036 x 1536: 106 -> 12 us; 512 x 768, r 8: 10 -> 6 us).
+// that it replaces read all of P for each token (2036 x 8960, r 16: 280 -> 36
+// us; 2036 x 1536: 106 -> 9 us; 512 x 768, r 8: 10 -> 5.5 us).
 // Every 16 products are summed on their own, the 16s in pairs, these per wave
 // and then the waves in order.
 template <int RT> constexpr int kF32RowWaves = RT <= 2 ? 16 : 8;  // 128 or 256 registers per lane
