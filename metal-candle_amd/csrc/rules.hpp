@@ -20,22 +20,24 @@ constexpr bool xent_wide_rows(int64_t rows, int64_t vocab, int elem_size) {
     return rows <= 256 ? vectors >= 1536 : rows <= 512 && vectors >= 6144;
 }
 
-// Gradients of the logits stored past the caches, once they are 96 MB of the 256
-// MB last-level cache. Below, logits and gradients both fit: there is little to
-// protect, and the product that reads the gradients finds them there. Above,
-// ordinary stores push out logits that the backward has yet to read. Time of
-// streamed over ordinary stores, logits not seen before: forward and backward
-// alone; with a pass over the gradients behind them; with a LoRA backward.
-//   50 MB   0.98-1.03  1.01-1.06  1.01-1.28
-//   95 MB   0.92-0.98  0.95-1.02  0.96-1.22
-//   115 MB  0.85-0.95  0.98-1.02  0.97-1.20
-//   145 MB  0.86-0.91  0.90-0.93  0.97-1.12 (bf16 0.97-0.98)
-//   300 MB  0.84-0.90  0.94-0.99  0.92-1.01
-// 2036 bf16 rows of 151936 (619 MB): 333 / 384 us alone, 562 / 577 with a pass,
-// 621 / 629 with a LoRA backward. From 900 MB on the two differ by less than 6%
-// either way.
+// Gradients of the logits stored past the caches, once they are 64 MB, a quarter
+// of the last-level cache. Below, the product that reads the gradients finds
+// them in the cache, and forward and backward alone lose nothing by it; above,
+// ordinary stores push out logits that the backward has yet to read, and more
+// of the next step's. Time of streamed over ordinary stores: forward and
+// backward in a loop over three inputs; on logits not seen before; followed by a
+// LoRA backward; between the product that made the logits and the one that
+// reads the gradients (torch.matmul, 896 features).
+//   20 MB   0.96-1.01  0.97-1.01  1.00-1.31  1.00-1.01
+//   50 MB   0.98-1.01  0.98-1.03  1.01-1.28  1.00-1.02
+//   85 MB   0.83-0.96  0.95-0.99  0.99-1.24  1.00 (70 MB, bf16 1.03)
+//   120 MB  0.77-0.86  0.82-0.95  0.97-1.18  1.00-1.01
+//   300 MB             0.84-0.90  0.92-1.01  0.98
+// 2036 bf16 rows of 151936 (619 MB), not seen before: 333 / 384 us, 621 / 629 with
+// a LoRA backward, 1685 / 1704 between products. From 900 MB on the two differ by
+// less than 6% either way.
 constexpr bool xent_stream_gradients(int64_t rows, int64_t vocab, int elem_size) {
-    return rows * vocab * elem_size > (int64_t)96 << 20;
+    return rows * vocab * elem_size > (int64_t)64 << 20;
 }
 
 // Softmax rows that are not whole 16-byte vectors: the covering vectors of the

@@ -167,25 +167,33 @@ def test_xent_wide_rows(rules, size, V, us):
         assert t[wide] <= 1.04 * min(t), rows
 
 
-# Cross-entropy forward and backward alone, and followed by a pass over the gradients, on logits not seen before,
-# us: ordinary stores, streamed.
-@pytest.mark.parametrize("size,rows,V,alone,followed", [
-    (4, 497, 50257, (63.3, 62.6), (92.2, 96.7)), (4, 781, 32000, (69.8, 64.6), (98.3, 100.5)),
-    (4, 164, 151936, (69.6, 62.6), (90.5, 91.5)), (4, 1093, 32000, (96.0, 82.2), (138.6, 128.7)),
-    (4, 795, 50257, (109.7, 99.0), (164.1, 150.6)), (4, 1492, 50257, (186.8, 157.6), (281.0, 265.5)),
-    (2, 994, 50257, (67.8, 65.5), (96.4, 100.2)), (2, 1562, 32000, (70.7, 65.1), (95.7, 100.7)),
-    (2, 460, 151936, (100.1, 88.3), (142.8, 128.7)), (2, 1989, 50257, (138.7, 119.6), (196.9, 187.4)),
-    (2, 2036, 151936, (384.4, 333.1), (577.3, 561.6)),
+# Cross-entropy forward and backward in a loop over three inputs, us: ordinary stores, streamed.
+@pytest.mark.parametrize("size,V,us", [
+    (4, 32000, {20: (25.7, 25.3), 50: (35.0, 35.2), 85: (55.3, 50.6), 100: (69.4, 61.8), 140: (95.2, 81.7)}),
+    (4, 151936, {20: (38.6, 38.7), 60: (41.5, 41.1), 70: (47.2, 42.4), 85: (55.8, 46.7), 120: (81.7, 63.5)}),
+    (2, 32000, {10: (25.2, 25.5), 50: (42.4, 42.3), 70: (45.9, 43.9), 100: (69.7, 60.1), 140: (101.3, 87.4)}),
+    (2, 151936, {20: (36.9, 35.5), 60: (39.6, 38.9), 85: (65.9, 63.1), 100: (77.2, 67.7), 140: (100.4, 87.1)}),
 ])
-def test_xent_stream_gradients(rules, size, rows, V, alone, followed):
+def test_xent_stream_gradients_alone(rules, size, V, us):
+    for mb, t in us.items():
+        stream = rules.xent_stream_gradients(ctypes.c_int64(mb * 10**6 // size // V), ctypes.c_int64(V), size)
+        assert t[stream] <= 1.04 * min(t), mb
+
+
+# The same on logits not seen before, with the LoRA backward that reads the gradients behind it, us.
+@pytest.mark.parametrize("size,rows,V,us", [
+    (4, 200, 32000, (129.9, 141.3)), (4, 200, 50257, (179.4, 234.6)), (4, 64, 151936, (487.5, 536.6)),
+    (2, 64, 32000, (143.7, 165.1)), (2, 500, 32000, (172.3, 187.5)), (2, 64, 151936, (559.6, 690.6)),
+    (2, 200, 151936, (656.3, 715.7)), (2, 1500, 151936, (492.1, 476.2)), (4, 4096, 8192, (143.6, 141.4)),
+])
+def test_xent_stream_gradients_with_reader(rules, size, rows, V, us):
     stream = rules.xent_stream_gradients(ctypes.c_int64(rows), ctypes.c_int64(V), size)
-    assert followed[stream] == min(followed)
-    assert alone[stream] <= 1.12 * min(alone)
+    assert us[stream] == min(us)
 
 
 def test_xent_stream_gradients_line(rules):
-    assert not rules.xent_stream_gradients(ctypes.c_int64(96 << 10), ctypes.c_int64(512), 2)
-    assert rules.xent_stream_gradients(ctypes.c_int64((96 << 10) + 1), ctypes.c_int64(512), 2)
+    assert not rules.xent_stream_gradients(ctypes.c_int64(64 << 10), ctypes.c_int64(512), 2)
+    assert rules.xent_stream_gradients(ctypes.c_int64((64 << 10) + 1), ctypes.c_int64(512), 2)
 
 
 def test_attention_f32_tiles_fit(rules):
